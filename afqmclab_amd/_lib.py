@@ -143,6 +143,10 @@ SIGNATURES = {
     "afqmc_ph_adjust_ET": (C.c_int, [_vp]),
     "afqmc_test_zgemm": (C.c_int, [_vp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _dp, C.c_longlong,
                                    _dp, _dp, C.c_int, C.c_int, C.c_int, _dp]),
+    "afqmc_test_real_gemm": (C.c_int, [_vp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _dp, _dp, _dp, C.c_int,
+                                       C.c_int, _dp]),
+    "afqmc_test_walker_panel": (C.c_int, [_vp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _dp, _dp, C.c_int, _ip,
+                                          _dp]),
     "afqmc_test_gj_inverse": (C.c_int, [_vp, C.c_int, C.c_int, C.c_int, _dp, _dp, _dp, _ip]),
     "afqmc_test_gj_inverse_layout": (C.c_int, [_vp, C.c_int, C.c_int, C.c_int, C.c_int, _dp, _dp, _dp, _ip]),
     "afqmc_test_gj_inverse_masked": (C.c_int, [_vp, C.c_int, C.c_int, C.c_int, C.c_int, _ip, _dp, _dp, _dp, _ip]),

@@ -28,6 +28,7 @@ struct afqmc_bp_s {
   DevBuf<int> tables;        // [max(nbp, 1)][nw]
   std::vector<char> has_table;
   std::vector<long long> snap_time;
+  std::vector<int> snap_real;  // afqmc_walkers_s::real of each copy
   std::vector<DevBuf<char>> snap;  // [nsnap * nblk]
   DevBuf<int> anc;
   afqmc_walkers bra = nullptr, ket = nullptr;
@@ -59,6 +60,7 @@ int snapshot_if_due(afqmc_bp bp, afqmc_walkers w) {
     HIP_TRY(hipMemcpyAsync(bp->snap[slot * cp->nblk + b].p, w->wf[b].p, cp->esz() * w->wsize(b) * w->nw,
                            hipMemcpyDeviceToDevice, cp->ctx->stream));
   bp->snap_time[slot] = bp->t;
+  bp->snap_real[slot] = w->real;
   return 0;
 }
 
@@ -75,11 +77,11 @@ int bra_step(afqmc_bp bp, afqmc_walkers bra, const int* aux, const int* table) {
   int rc = launch_bp_field(f, s);
   if (rc) return rc;
   if (cp->diag_only) {
-    if ((rc = propagate_gemm<T>(cp, bra, 0, bra->wf, bra->tmp, true))) return rc;
+    if ((rc = propagate_gemm<T>(cp, bra, 0, bra->wf, bra->tmp, true, bra->real))) return rc;
   } else {
     if ((rc = launch_hs_apply_2x2<T>(bp->nw, cp->L, cp->N, bra->wf[0].p, bra->tmp[0].p, cp->d2x2.p, s))) return rc;
     std::swap(bra->wf[0], bra->tmp[0]);
-    if ((rc = propagate_gemm<T>(cp, bra, 0, bra->wf, bra->tmp, false))) return rc;
+    if ((rc = propagate_gemm<T>(cp, bra, 0, bra->wf, bra->tmp, false, bra->real))) return rc;
   }
   for (int b = 0; b < cp->nblk; ++b) std::swap(bra->wf[b], bra->tmp[b]);
   return 0;
@@ -93,6 +95,9 @@ int measure_impl(afqmc_bp bp, afqmc_walkers w, int snap_slot) {
   afqmc_walkers bra = bp->bra, ket = bp->ket;
   const int nw = bp->nw, L = cp->L;
   int rc;
+  // the bras come from the trial; the kets are as real as the walkers were when they were copied
+  bra->real = cp->real_ops;
+  ket->real = bp->snap_real[snap_slot];
   // weights: the mixed overlaps of the current walkers
   if ((rc = mixed_weight(cp, w))) return rc;
   HIP_TRY(hipMemcpyAsync(bra->alive.p, w->alive.p, sizeof(int) * nw, hipMemcpyDeviceToDevice, s));
@@ -102,7 +107,7 @@ int measure_impl(afqmc_bp bp, afqmc_walkers w, int snap_slot) {
   for (int b = 0; b < cp->nblk; ++b)
     if ((rc = launch_gather_walkers(nw, bra->wsize(b), cp->esz(), nullptr, cp->phiT[b].p, bra->tmp[b].p, s)))
       return rc;
-  if ((rc = propagate_gemm<T>(cp, bra, 1, bra->tmp, bra->wf, false))) return rc;
+  if ((rc = propagate_gemm<T>(cp, bra, 1, bra->tmp, bra->wf, false, bra->real))) return rc;
   // the recorded steps, last first: D^H then exp(-dt K)^H, normalised every mgs steps
   const long long start = bp->t - bp->nbp;
   for (int j = bp->nbp - 1; j >= 0; --j) {
@@ -113,14 +118,14 @@ int measure_impl(afqmc_bp bp, afqmc_walkers w, int snap_slot) {
     if ((bp->nbp - j) % bp->mgs == 0 && (rc = stabilize(cp, bra))) return rc;
   }
   // bra = exp(dt/2 K)^H bra, ket = exp(dt/2 K) backup[anc]
-  if ((rc = propagate_gemm<T>(cp, bra, 2, bra->wf, bra->tmp, false))) return rc;
+  if ((rc = propagate_gemm<T>(cp, bra, 2, bra->wf, bra->tmp, false, bra->real))) return rc;
   for (int b = 0; b < cp->nblk; ++b) {
     std::swap(bra->wf[b], bra->tmp[b]);
     if ((rc = launch_gather_walkers(nw, ket->wsize(b), cp->esz(), bp->anc.p, bp->snap[snap_slot * cp->nblk + b].p,
                                     ket->tmp[b].p, s)))
       return rc;
   }
-  if ((rc = propagate_gemm<T>(cp, ket, 2, ket->tmp, ket->wf, false))) return rc;
+  if ((rc = propagate_gemm<T>(cp, ket, 2, ket->tmp, ket->wf, false, ket->real))) return rc;
   // per block: S = bra^H ket, S^{-1}, Theta = ket S^{-1} (into bra->tmp), bra^H (into ket->tmp)
   for (int b = 0; b < cp->nblk; ++b) {
     const int Mb = cp->Mb[b], Nb = cp->Nb[b];
@@ -196,6 +201,7 @@ int afqmc_bp_create(afqmc_cp cp, int nw, int bp_steps, int measure_skip, int mgs
   if (!rc) rc = bp->tables.alloc(ring * nw);
   bp->has_table.assign(ring, 0);
   bp->snap_time.assign(bp->nsnap, -1);
+  bp->snap_real.assign(bp->nsnap, 0);
   bp->snap.resize((size_t)bp->nsnap * cp->nblk);
   long long wbytes = 0;
   for (int b = 0; b < cp->nblk; ++b) wbytes += (long long)cp->Mb[b] * cp->Nb[b];

@@ -77,7 +77,7 @@ LogOArgs logo_args(afqmc_cp cp, afqmc_walkers w, int mode) {
 
 template <typename T>
 int do_overlap(afqmc_cp cp, afqmc_walkers w, bool inverse) {
-  int rc = overlap_gemm<T>(cp, w, w->wf);
+  int rc = overlap_gemm<T>(cp, w, w->wf, w->real);
   if (!rc) rc = gj_blocks<T>(cp, w, inverse, w->alive.p);
   return rc;
 }
@@ -111,7 +111,7 @@ int step_impl(afqmc_cp cp, afqmc_walkers w, double* force_out, int* aux_out, int
   for (int b = 0; b < cp->nblk; ++b) capture_note_pair(&w->wf[b], &w->tmp[b]);
   {
     RegionTimer t(cp->ctx, REG_OVERLAP);
-    if ((rc = overlap_gemm<T>(cp, w, w->wf))) return rc;
+    if ((rc = overlap_gemm<T>(cp, w, w->wf, w->real))) return rc;
   }
   {
     RegionTimer t(cp->ctx, REG_GJ);
@@ -122,7 +122,7 @@ int step_impl(afqmc_cp cp, afqmc_walkers w, double* force_out, int* aux_out, int
   if ((rc = launch_alive_scan(w->nw, w->alive.p, cp->prefix.p, cp->sc.p, s))) return rc;
   {
     RegionTimer t(cp->ctx, REG_GREEN);
-    if ((rc = green_gemm<T>(cp, w, w->wf, w->alive.p, false))) return rc;
+    if ((rc = green_gemm<T>(cp, w, w->wf, w->alive.p, false, w->real))) return rc;
   }
   HsSampleArgs h = hs_args<T>(cp, w);
   if (force_out || aux_out) {
@@ -139,7 +139,7 @@ int step_impl(afqmc_cp cp, afqmc_walkers w, double* force_out, int* aux_out, int
   }
   if (cp->diag_only) {
     RegionTimer t(cp->ctx, REG_PROPAGATE);
-    if ((rc = propagate_gemm<T>(cp, w, 0, w->wf, w->tmp, true))) return rc;
+    if ((rc = propagate_gemm<T>(cp, w, 0, w->wf, w->tmp, true, w->real))) return rc;
   } else {
     {
       RegionTimer t(cp->ctx, REG_HS_APPLY);
@@ -147,7 +147,7 @@ int step_impl(afqmc_cp cp, afqmc_walkers w, double* force_out, int* aux_out, int
     }
     for (int b = 0; b < cp->nblk; ++b) std::swap(w->wf[b], w->tmp[b]);
     RegionTimer t(cp->ctx, REG_PROPAGATE);
-    if ((rc = propagate_gemm<T>(cp, w, 0, w->wf, w->tmp, false))) return rc;
+    if ((rc = propagate_gemm<T>(cp, w, 0, w->wf, w->tmp, false, w->real))) return rc;
   }
   // the propagated walkers are in tmp: make them current
   for (int b = 0; b < cp->nblk; ++b) std::swap(w->wf[b], w->tmp[b]);
@@ -272,14 +272,14 @@ int measure_impl(afqmc_cp cp, afqmc_walkers w) {
   hipStream_t s = cp->ctx->stream;
   RegionTimer t(cp->ctx, REG_MEASURE);
   int rc;
-  if ((rc = propagate_gemm<T>(cp, w, 2, w->wf, w->tmp, false))) return rc;
+  if ((rc = propagate_gemm<T>(cp, w, 2, w->wf, w->tmp, false, w->real))) return rc;
   if ((rc = launch_logw_shift(w->nw, w->logw.p, w->logw_tmp.p, cp->hop_logw[2], s))) return rc;
-  if ((rc = overlap_gemm<T>(cp, w, w->tmp))) return rc;
+  if ((rc = overlap_gemm<T>(cp, w, w->tmp, w->real))) return rc;
   if ((rc = gj_blocks<T>(cp, w, true, w->alive.p))) return rc;
   LogOArgs l = logo_args<T>(cp, w, LOGO_MEASURE);
   l.logw = w->logw_tmp.p;
   if ((rc = launch_logo(l, s))) return rc;
-  if ((rc = green_gemm<T>(cp, w, w->tmp, w->alive.p, true))) return rc;
+  if ((rc = green_gemm<T>(cp, w, w->tmp, w->alive.p, true, w->real))) return rc;
   EnergyArgs e;
   memset(&e, 0, sizeof(e));
   e.nw = w->nw; e.L = cp->L; e.nblk = cp->nblk; e.dense = cp->dense;
@@ -298,9 +298,9 @@ template <typename T>
 int mixed_weight_impl(afqmc_cp cp, afqmc_walkers w) {
   hipStream_t s = cp->ctx->stream;
   int rc;
-  if ((rc = propagate_gemm<T>(cp, w, 2, w->wf, w->tmp, false))) return rc;
+  if ((rc = propagate_gemm<T>(cp, w, 2, w->wf, w->tmp, false, w->real))) return rc;
   if ((rc = launch_logw_shift(w->nw, w->logw.p, w->logw_tmp.p, cp->hop_logw[2], s))) return rc;
-  if ((rc = overlap_gemm<T>(cp, w, w->tmp))) return rc;
+  if ((rc = overlap_gemm<T>(cp, w, w->tmp, w->real))) return rc;
   if ((rc = gj_blocks<T>(cp, w, false, w->alive.p))) return rc;
   LogOArgs l = logo_args<T>(cp, w, LOGO_MEASURE);
   l.logw = w->logw_tmp.p;
@@ -334,9 +334,9 @@ int tune_role(afqmc_cp cp, afqmc_walkers w, int role, int reps, double* ms_row) 
     cp->tile[role] = t;
     auto run = [&]() {
       // each role reads the walkers and writes only workspace (tmp, overlaps, Green partials)
-      if (role == 0) return propagate_gemm<T>(cp, w, 0, w->wf, w->tmp, cp->diag_only != 0);
-      if (role == 1) return overlap_gemm<T>(cp, w, w->wf);
-      return green_gemm<T>(cp, w, w->wf, w->alive.p, false);
+      if (role == 0) return propagate_gemm<T>(cp, w, 0, w->wf, w->tmp, cp->diag_only != 0, w->real);
+      if (role == 1) return overlap_gemm<T>(cp, w, w->wf, w->real);
+      return green_gemm<T>(cp, w, w->wf, w->alive.p, false, w->real);
     };
     if ((rc = run())) break;
     if (hipEventRecord(e0, s) != hipSuccess) { rc = -2; break; }
@@ -468,6 +468,18 @@ int afqmc_cp_create(afqmc_ctx ctx, const afqmc_cp_desc* d, afqmc_cp* out) {
       if (!rc) rc = upload_matrix_blocks<double>(cp, (const double*)wdkT.data(), d->N, cp->wdkT, false);
     }
   }
+  // real operators: kept as real arrays too
+  if (!rc) {
+    bool real_wdk = false;
+    const double* wdk = (const double*)wdkT.data();
+    rc = cp->fp32 ? upload_real_operators<float>(cp, d->phiT, mats, wdk, &real_wdk)
+                  : upload_real_operators<double>(cp, d->phiT, mats, wdk, &real_wdk);
+    auto zero_im = [](const std::vector<cd>& v) {
+      return std::all_of(v.begin(), v.end(), [](const cd& z) { return z.imag() == 0.0 && std::isfinite(z.real()); });
+    };
+    cp->real_ops = cp->real_phi && cp->real_expk[0] && cp->real_expk[1] && cp->real_expk[2] && zero_im(K) &&
+                   real_wdk && zero_im(cp->h_gamma) && zero_im(cp->h_cdiag);
+  }
   // workspace
   const int nw = d->max_walkers;
   const size_t es = cp->esz();
@@ -549,6 +561,7 @@ int afqmc_cp_walkers_create(afqmc_cp cp, int nw, afqmc_walkers* out) {
   w->cp = cp;
   w->device = cp->device;
   w->nw = nw;
+  w->real = cp->real_ops;  // zeros
   int rc = 0;
   for (int b = 0; b < cp->nblk && !rc; ++b) {
     rc = w->wf[b].alloc_bytes(cp->esz() * w->wsize(b) * nw);
@@ -604,20 +617,26 @@ int afqmc_walkers_upload(afqmc_walkers w, const double* wf, const double* logw, 
           }
         }
   }
+  const int keep_real = cp->real_ops;
+  w->real = 0;  // until every element has been looked at
+  bool real = true;
   for (int b = 0; b < cp->nblk; ++b) {
     const long long ws = w->wsize(b);
     if (cp->fp32) {
       std::vector<zf> h(ws * w->nw);
       for (int iw = 0; iw < w->nw; ++iw)
         pack_block<float>(wf + 2 * iw * per, L2, N, cp->row0[b], cp->col0[b], cp->Mb[b], cp->Nb[b], h, iw * ws);
+      real = real && keep_real && all_real(h.data(), h.size());
       HIP_TRY(hipMemcpy(w->wf[b].p, h.data(), sizeof(zf) * h.size(), hipMemcpyHostToDevice));
     } else {
       std::vector<zd> h(ws * w->nw);
       for (int iw = 0; iw < w->nw; ++iw)
         pack_block<double>(wf + 2 * iw * per, L2, N, cp->row0[b], cp->col0[b], cp->Mb[b], cp->Nb[b], h, iw * ws);
+      real = real && keep_real && all_real(h.data(), h.size());
       HIP_TRY(hipMemcpy(w->wf[b].p, h.data(), sizeof(zd) * h.size(), hipMemcpyHostToDevice));
     }
   }
+  w->real = real && keep_real;
   HIP_TRY(hipMemcpy(w->logw.p, logw, sizeof(zd) * w->nw, hipMemcpyHostToDevice));
   std::vector<int> a(w->nw, 1);
   if (alive) std::copy(alive, alive + w->nw, a.begin());
@@ -725,6 +744,7 @@ int afqmc_cp_walkers_from_trial(afqmc_cp cp, afqmc_walkers w, const double* logw
   ScopedDevice sd(cp->ctx);
   hipStream_t s = cp->ctx->stream;
   HIP_TRY(hipStreamSynchronize(s));
+  w->real = cp->real_ops;
   // phiT into walker 0, then doubling device copies [0, k) -> [k, 2k)
   for (int b = 0; b < cp->nblk; ++b) {
     const size_t bytes = cp->esz() * (size_t)w->wsize(b);
@@ -861,8 +881,8 @@ int afqmc_cp_green_diagonal(afqmc_cp cp, afqmc_walkers w, double* gdiag, double*
   REQUIRE(cp && w && gdiag && w->cp == cp, "invalid argument");
   ScopedDevice sd(cp->ctx);
   int rc = cp->fp32 ? do_overlap<float>(cp, w, true) : do_overlap<double>(cp, w, true);
-  if (!rc) rc = cp->fp32 ? green_gemm<float>(cp, w, w->wf, w->alive.p, false)
-                         : green_gemm<double>(cp, w, w->wf, w->alive.p, false);
+  if (!rc) rc = cp->fp32 ? green_gemm<float>(cp, w, w->wf, w->alive.p, false, w->real)
+                         : green_gemm<double>(cp, w, w->wf, w->alive.p, false, w->real);
   if (rc) return rc;
   HIP_TRY(hipStreamSynchronize(cp->ctx->stream));
   const int L = cp->L, L2 = 2 * L;
@@ -924,8 +944,8 @@ int afqmc_cp_onebody(afqmc_cp cp, afqmc_walkers w, int which) {
   REQUIRE(cp && w && w->cp == cp, "invalid argument");
   REQUIRE(which >= 0 && which <= 2, "which must be 0, 1 or 2");
   ScopedDevice sd(cp->ctx);
-  int rc = cp->fp32 ? propagate_gemm<float>(cp, w, which, w->wf, w->tmp, false)
-                    : propagate_gemm<double>(cp, w, which, w->wf, w->tmp, false);
+  int rc = cp->fp32 ? propagate_gemm<float>(cp, w, which, w->wf, w->tmp, false, w->real)
+                    : propagate_gemm<double>(cp, w, which, w->wf, w->tmp, false, w->real);
   if (rc) return rc;
   // alive walkers take the product, killed ones keep their state (the reference skips them)
   for (int b = 0; b < cp->nblk; ++b) {
@@ -934,6 +954,8 @@ int afqmc_cp_onebody(afqmc_cp cp, afqmc_walkers w, int which) {
   }
   if ((rc = launch_logw_const_add(w->nw, w->logw.p, w->alive.p, cp->hop_logw[which], cp->ctx->stream))) return rc;
   HIP_TRY(sync_unless_capturing(cp->ctx->stream));
+  capture_note_real(&w->real);
+  capture_note_call([=] { return afqmc_cp_onebody(cp, w, which); });
   return 0;
 }
 
@@ -946,6 +968,8 @@ int afqmc_cp_hs_apply(afqmc_cp cp, afqmc_walkers w, const double* diag4, const d
   const int L = cp->L;
   const size_t n = (size_t)4 * L * w->nw;
   int rc = 0;
+  // real walkers stay real under real site matrices only
+  if (w->real && !all_real(reinterpret_cast<const zd*>(diag4), n)) w->real = 0;
   DevBuf<char> d;
   if ((rc = d.alloc_bytes(cp->esz() * n))) return rc;
   if (cp->fp32) {
@@ -975,6 +999,8 @@ int afqmc_cp_stabilize(afqmc_cp cp, afqmc_walkers w) {
   int rc = stabilize_impl(cp, w);
   if (rc) return rc;
   HIP_TRY(sync_unless_capturing(cp->ctx->stream));
+  capture_note_real(&w->real);
+  capture_note_call([=] { return afqmc_cp_stabilize(cp, w); });
   return 0;
 }
 
@@ -1026,14 +1052,22 @@ int afqmc_cp_apply_table(afqmc_cp cp, afqmc_walkers w, const int* table) {
 int afqmc_cp_step(afqmc_cp cp, afqmc_walkers w, double* force_out, int* aux_out) {
   REQUIRE(cp && w && w->cp == cp, "invalid argument");
   ScopedDevice sd(cp->ctx);
-  return DISPATCH(cp, step_impl, cp, w, force_out, aux_out);
+  int rc = DISPATCH(cp, step_impl, cp, w, force_out, aux_out);
+  if (rc) return rc;
+  capture_note_real(&w->real);
+  capture_note_call([=] { return afqmc_cp_step(cp, w, nullptr, nullptr); });
+  return 0;
 }
 
 int afqmc_cp_pop_control(afqmc_cp cp, afqmc_walkers w, double* weights_out, int* table_out, double* stats) {
   REQUIRE(cp && w && w->cp == cp, "invalid argument");
   REQUIRE(!capturing() || (!weights_out && !table_out && !stats), "a captured comb cannot return outputs");
   ScopedDevice sd(cp->ctx);
-  return DISPATCH(cp, pop_control_impl, cp, w, weights_out, table_out, stats);
+  int rc = DISPATCH(cp, pop_control_impl, cp, w, weights_out, table_out, stats);
+  if (rc) return rc;
+  capture_note_real(&w->real);
+  capture_note_call([=] { return afqmc_cp_pop_control(cp, w, nullptr, nullptr, nullptr); });
+  return 0;
 }
 
 int afqmc_cp_step_fields(afqmc_cp cp, afqmc_walkers w, const int* aux) {
@@ -1080,7 +1114,11 @@ int afqmc_cp_pop_control_table(afqmc_cp cp, afqmc_walkers w, const int* table, d
 int afqmc_cp_measure(afqmc_cp cp, afqmc_walkers w) {
   REQUIRE(cp && w && w->cp == cp, "invalid argument");
   ScopedDevice sd(cp->ctx);
-  return DISPATCH(cp, measure_impl, cp, w);
+  int rc = DISPATCH(cp, measure_impl, cp, w);
+  if (rc) return rc;
+  capture_note_real(&w->real);
+  capture_note_call([=] { return afqmc_cp_measure(cp, w); });
+  return 0;
 }
 
 int afqmc_cp_energy(afqmc_cp cp, double* out) {
@@ -1109,6 +1147,7 @@ int afqmc_cp_reset_measure(afqmc_cp cp) {
   ScopedDevice sd(cp->ctx);
   int rc = launch_reset_measure(cp->sc.p, cp->site_acc.p, cp->L, cp->ctx->stream);
   if (rc) return rc;
+  capture_note_call([=] { return afqmc_cp_reset_measure(cp); });
   return 0;
 }
 
@@ -1116,8 +1155,10 @@ int afqmc_cp_adjust_ET(afqmc_cp cp) {
   REQUIRE(cp, "null argument");
   ScopedDevice sd(cp->ctx);
   int rc = launch_set_et_from_energy(cp->sc.p, cp->ctx->stream);
+  if (!rc) rc = launch_reset_measure(cp->sc.p, cp->site_acc.p, cp->L, cp->ctx->stream);
   if (rc) return rc;
-  return launch_reset_measure(cp->sc.p, cp->site_acc.p, cp->L, cp->ctx->stream);
+  capture_note_call([=] { return afqmc_cp_adjust_ET(cp); });
+  return 0;
 }
 
 int afqmc_cp_set_tiles(afqmc_cp cp, const int* tiles) {
@@ -1186,8 +1227,10 @@ int run_grouped(afqmc_cp_group g, F&& per_member) {
   g_group = nullptr;
   for (size_t i = 0; i < n; ++i)
     for (int r = 0; r < 3; ++r) g->cps[i]->tile[r] = saved[i][r];
+  if (!rc) rc = group_flush_all(c, g->ctx->stream);
   if (rc) return rc;
-  return group_flush_all(c, g->ctx->stream);
+  for (afqmc_walkers w : g->ws) capture_note_real(&w->real);
+  return 0;
 }
 
 }  // namespace
@@ -1230,22 +1273,28 @@ int afqmc_cp_group_set_tiles(afqmc_cp_group g, const int* tiles) {
 
 int afqmc_cp_group_step(afqmc_cp_group g) {
   REQUIRE(g, "null argument");
-  return run_grouped(g, [&](afqmc_cp cp, afqmc_walkers w) {
+  int rc = run_grouped(g, [&](afqmc_cp cp, afqmc_walkers w) {
     return g->fp32 ? step_impl<float>(cp, w, nullptr, nullptr) : step_impl<double>(cp, w, nullptr, nullptr);
   });
+  if (!rc) capture_note_call([=] { return afqmc_cp_group_step(g); });
+  return rc;
 }
 
 int afqmc_cp_group_stabilize(afqmc_cp_group g) {
   REQUIRE(g, "null argument");
-  return run_grouped(g, [&](afqmc_cp cp, afqmc_walkers w) { return stabilize_impl(cp, w); });
+  int rc = run_grouped(g, [&](afqmc_cp cp, afqmc_walkers w) { return stabilize_impl(cp, w); });
+  if (!rc) capture_note_call([=] { return afqmc_cp_group_stabilize(g); });
+  return rc;
 }
 
 int afqmc_cp_group_pop_control(afqmc_cp_group g) {
   REQUIRE(g, "null argument");
-  return run_grouped(g, [&](afqmc_cp cp, afqmc_walkers w) {
+  int rc = run_grouped(g, [&](afqmc_cp cp, afqmc_walkers w) {
     return g->fp32 ? pop_control_impl<float>(cp, w, nullptr, nullptr, nullptr)
                    : pop_control_impl<double>(cp, w, nullptr, nullptr, nullptr);
   });
+  if (!rc) capture_note_call([=] { return afqmc_cp_group_pop_control(g); });
+  return rc;
 }
 
 int afqmc_cp_group_table_count(afqmc_cp_group g) { return g ? (int)g->tables.count() : -1; }

@@ -5,8 +5,10 @@
 #include <vector>
 
 #include "gemm.hpp"
+#include "real_gemm.hpp"
 #include "runtime.hpp"
 #include "small_dense.hpp"
+#include "walker_panel.hpp"
 
 namespace {
 
@@ -111,9 +113,100 @@ int gj_t(afqmc_ctx ctx, int kind, int N, int batch, const double* A, double* Ain
   return 0;
 }
 
+template <typename T>
+int real_gemm_t(afqmc_ctx ctx, int op_t, int M, int N, int K, const double* A, const double* B, const double* scale,
+                int scale_group, int b_real, double* C) {
+  hipStream_t s = ctx->stream;
+  const size_t nA = (size_t)M * K, nB = (size_t)K * N, nC = (size_t)M * N;
+  std::vector<T> hA(A, A + nA);
+  auto hB = narrow<T>(B, nB);
+  DevBuf<T> dA;
+  DevBuf<cplx<T>> dB, dC, dS;
+  int rc = dA.alloc(nA);
+  if (!rc) rc = dB.alloc(nB);
+  if (!rc) rc = dC.alloc(nC);
+  if (rc) return rc;
+  HIP_TRY(hipMemcpy(dA.p, hA.data(), sizeof(T) * nA, hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(dB.p, hB.data(), sizeof(cplx<T>) * nB, hipMemcpyHostToDevice));
+  RealGemmArgs a;
+  memset(&a, 0, sizeof(a));
+  a.M = M; a.N = N; a.K = K; a.op_t = op_t; a.alpha = 1.0; a.b_real = b_real;
+  a.A = dA.p; a.lda = op_t ? K : M; a.B = dB.p; a.ldb = K; a.C = dC.p; a.ldc = M;
+  if (scale) {
+    const size_t nS = (size_t)K * ((N + scale_group - 1) / scale_group);
+    auto hS = narrow<T>(scale, nS);
+    if ((rc = dS.alloc(nS))) return rc;
+    HIP_TRY(hipMemcpy(dS.p, hS.data(), sizeof(cplx<T>) * nS, hipMemcpyHostToDevice));
+    a.scale = dS.p; a.scale_group = scale_group; a.scale_strideG = K;
+  }
+  if ((rc = launch_real_gemm<T>(a, s))) return rc;
+  std::vector<cplx<T>> hC(nC);
+  HIP_TRY(hipMemcpyAsync(hC.data(), dC.p, sizeof(cplx<T>) * nC, hipMemcpyDeviceToHost, s));
+  HIP_TRY(hipStreamSynchronize(s));
+  for (size_t i = 0; i < nC; ++i) { C[2 * i] = hC[i].re; C[2 * i + 1] = hC[i].im; }
+  return 0;
+}
+
+// what: 1 W B, 2 W^T W; TS the walkers' type, TC the type of B and of the Gram matrix
+template <typename TS, typename TC>
+int panel_t(afqmc_ctx ctx, int what, int M, int N, int nw, const double* W, const double* B, int b_upper,
+            const int* alive, double* out) {
+  hipStream_t s = ctx->stream;
+  const size_t nW = (size_t)M * N * nw, nB = (size_t)N * N * nw;
+  auto hW = narrow<TS>(W, nW);
+  DevBuf<cplx<TS>> dW;
+  DevBuf<cplx<TC>> dB;
+  DevBuf<int> al;
+  int rc = dW.alloc(nW);
+  if (!rc) rc = dB.alloc(nB);
+  if (!rc) rc = al.alloc(nw);
+  if (rc) return rc;
+  HIP_TRY(hipMemcpy(dW.p, hW.data(), sizeof(cplx<TS>) * nW, hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(al.p, alive, sizeof(int) * nw, hipMemcpyHostToDevice));
+  std::vector<cplx<TC>> hB(nB, cmk<TC>(0, 0));
+  if (what == 1) hB = narrow<TC>(B, nB);
+  HIP_TRY(hipMemcpy(dB.p, hB.data(), sizeof(cplx<TC>) * nB, hipMemcpyHostToDevice));
+  WalkerPanelArgs a;
+  memset(&a, 0, sizeof(a));
+  a.M = M; a.N = N; a.nw = nw; a.W = dW.p; a.strideW = (long long)M * N; a.alive = al.p;
+  if (what == 1) {
+    a.B = dB.p; a.strideB = (long long)N * N; a.b_upper = b_upper;
+    a.out = dW.p; a.stride_out = a.strideW;  // in place
+    if ((rc = launch_walker_times<TS, TC>(a, s))) return rc;
+    HIP_TRY(hipMemcpyAsync(hW.data(), dW.p, sizeof(cplx<TS>) * nW, hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    for (size_t i = 0; i < nW; ++i) { out[2 * i] = hW[i].re; out[2 * i + 1] = hW[i].im; }
+  } else {
+    a.out = dB.p; a.stride_out = (long long)N * N;
+    if ((rc = launch_walker_gram<TS, TC>(a, s))) return rc;
+    HIP_TRY(hipMemcpyAsync(hB.data(), dB.p, sizeof(cplx<TC>) * nB, hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    for (size_t i = 0; i < nB; ++i) { out[2 * i] = hB[i].re; out[2 * i + 1] = hB[i].im; }
+  }
+  return 0;
+}
+
 }  // namespace
 
 extern "C" {
+
+int afqmc_test_real_gemm(afqmc_ctx ctx, int precision, int op_t, int M, int N, int K, const double* A, const double* B,
+                         const double* scale, int scale_group, int b_real, double* C) {
+  REQUIRE(ctx && A && B && C, "null argument");
+  REQUIRE(M > 0 && N > 0 && K > 0 && (!scale || (!op_t && scale_group > 0)), "invalid sizes");
+  ScopedDevice sd(ctx);
+  return precision ? real_gemm_t<float>(ctx, op_t, M, N, K, A, B, scale, scale_group, b_real, C)
+                   : real_gemm_t<double>(ctx, op_t, M, N, K, A, B, scale, scale_group, b_real, C);
+}
+
+int afqmc_test_walker_panel(afqmc_ctx ctx, int precision, int what, int M, int N, int nw, const double* W,
+                            const double* B, int b_upper, const int* alive, double* out) {
+  REQUIRE(ctx && W && alive && out && (what == 2 || (what == 1 && B)), "invalid argument");
+  REQUIRE(M > 0 && N > 0 && nw > 0 && precision >= 0 && precision <= 1, "invalid sizes");
+  ScopedDevice sd(ctx);
+  return precision ? panel_t<float, double>(ctx, what, M, N, nw, W, B, b_upper, alive, out)
+                   : panel_t<double, double>(ctx, what, M, N, nw, W, B, b_upper, alive, out);
+}
 
 int afqmc_test_zgemm(afqmc_ctx ctx, int precision, int opa, int M, int N, int K, int batch, const double* A,
                      long long strideA, const double* B, const double* scale, int scale_group, int flags, int tile,

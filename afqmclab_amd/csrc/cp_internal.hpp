@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <complex>
 #include <type_traits>
 #include <cstring>
@@ -12,8 +13,10 @@
 #include "cp_kernels.hpp"
 #include "gemm.hpp"
 #include "group.hpp"
+#include "real_gemm.hpp"
 #include "runtime.hpp"
 #include "small_dense.hpp"
+#include "walker_panel.hpp"
 
 using cd = std::complex<double>;
 
@@ -28,6 +31,13 @@ struct afqmc_cp_s {
   zd trial_logw{0, 0};
   zd hop_logw[3];
   DevBuf<char> phiT[2], expK[3][2], wdkT[2];
+  // Operators whose imaginary parts are all zero, found once at creation: the trial and the
+  // propagators are then kept as real arrays too and their products take real_gemm.  real_ops: all
+  // of them, K, gamma and the site constants are real, so that walkers stay real under every
+  // operation of this propagator (afqmc_walkers_s::real).
+  int real_phi = 0, real_expk[3] = {0, 0, 0}, real_ops = 0;
+  DevBuf<char> real_buf;  // holds:
+  char *phiTr[2] = {}, *expKr[3][2] = {}, *wdkTr[2] = {};
   DevBuf<zd> gamma, cdiag;
   DevBuf<double> U, mu, hx, hy, hz, cforce;
   DevBuf<DevScalars> sc;
@@ -54,6 +64,9 @@ struct afqmc_walkers_s {
   DevBuf<char> wf[2], tmp[2];
   DevBuf<zd> logw, logw_tmp;
   DevBuf<int> alive;
+  // the imaginary part of every walker element is zero: set where the host knows what it writes
+  // (creation, upload, trial), kept by every operation of a propagator with real_ops
+  int real = 0;
   long long wsize(int b) const { return (long long)cp->Mb[b] * cp->Nb[b]; }
 };
 
@@ -68,6 +81,14 @@ void pack_block(const double* dense, int L2, int N, int r0, int c0, int Mb, int 
       const double* s = dense + 2 * ((long long)(r0 + i) + (long long)(c0 + j) * L2);
       out[off + i + (long long)j * Mb] = cmk<T>((T)s[0], (T)s[1]);
     }
+}
+
+// every imaginary part zero and every real part finite
+template <typename T>
+bool all_real(const cplx<T>* v, size_t n) {
+  bool ok = true;
+  for (size_t k = 0; k < n; ++k) ok = ok && v[k].im == (T)0 && std::isfinite(v[k].re);
+  return ok;
 }
 
 template <typename T>
@@ -99,12 +120,69 @@ int cp_gemm(afqmc_cp cp, int opa, int epi, const GemmArgs& a) {
   return launch_cgemm<T>(opa, epi, a, cp->ctx->stream);
 }
 
-// overlap O_b = phiT_b^H W_b for all walkers ("giant" GEMM with shared A)
+// the matrix blocks' real parts appended to `out` (each block at a multiple of 16 bytes, its offset
+// in off[b]) when every imaginary part is zero and every real part finite in T; else nothing
 template <typename T>
-int overlap_gemm(afqmc_cp cp, afqmc_walkers w, DevBuf<char>* wf) {
+bool append_real_blocks(afqmc_cp cp, const double* dense, int cols, bool square, std::vector<T>& out, size_t* off) {
+  const int L2 = 2 * cp->L;
+  std::vector<cplx<T>> h[2];
+  for (int b = 0; b < cp->nblk; ++b) {
+    const int Mb = cp->Mb[b], Nb = square ? cp->Mb[b] : cp->Nb[b];
+    h[b].resize((size_t)Mb * Nb);
+    pack_block<T>(dense, L2, cols, cp->row0[b], square ? cp->row0[b] : cp->col0[b], Mb, Nb, h[b], 0);
+    if (!all_real(h[b].data(), h[b].size())) return false;
+  }
+  for (int b = 0; b < cp->nblk; ++b) {
+    out.resize((out.size() + 3) / 4 * 4);
+    off[b] = out.size();
+    for (const cplx<T>& v : h[b]) out.push_back(v.re);
+  }
+  return true;
+}
+
+// The real copies of the trial, the propagators and (phiT^H K)^T, in one device buffer; sets real_phi,
+// real_expk and *real_wdk.
+template <typename T>
+int upload_real_operators(afqmc_cp cp, const double* phiT, const double* const* mats, const double* wdkT, bool* real_wdk) {
+  std::vector<T> h;
+  size_t off[5][2] = {};
+  cp->real_phi = append_real_blocks<T>(cp, phiT, cp->N, false, h, off[0]);
+  for (int k = 0; k < 3; ++k) cp->real_expk[k] = append_real_blocks<T>(cp, mats[k], 2 * cp->L, true, h, off[1 + k]);
+  *real_wdk = append_real_blocks<T>(cp, wdkT, cp->N, false, h, off[4]);
+  if (h.empty()) return 0;
+  int rc = cp->real_buf.alloc_bytes(h.size() * sizeof(T));
+  if (rc) return rc;
+  HIP_TRY(hipMemcpy(cp->real_buf.p, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
+  for (int b = 0; b < cp->nblk; ++b) {
+    auto at = [&](int k) { return cp->real_buf.p + off[k][b] * sizeof(T); };
+    cp->phiTr[b] = at(0);
+    for (int k = 0; k < 3; ++k) cp->expKr[k][b] = at(1 + k);
+    cp->wdkTr[b] = at(4);
+  }
+  return 0;
+}
+
+// overlap O_b = phiT_b^H W_b for all walkers ("giant" GEMM with shared A).  real: the imaginary
+// parts of wf are zero.  A real trial takes real products (two per complex B element, one per
+// real one, against three in FP32 and four in FP64).
+template <typename T>
+int overlap_gemm(afqmc_cp cp, afqmc_walkers w, DevBuf<char>* wf, int real = 0) {
   GroupFork fork;  // the blocks are independent: a grouped call launches them together
   for (int b = 0; b < cp->nblk; ++b) {
     fork.branch();
+    if (cp->real_phi) {
+      RealGemmArgs r;
+      memset(&r, 0, sizeof(r));
+      r.M = cp->Nb[b]; r.N = cp->Nb[b] * w->nw; r.K = cp->Mb[b]; r.op_t = 1; r.alpha = 1.0; r.b_real = real;
+      r.A = cp->phiTr[b]; r.lda = cp->Mb[b];
+      r.B = wf[b].p; r.ldb = cp->Mb[b];
+      r.C = cp->ovl[b].p; r.ldc = cp->Nb[b];
+      if (real_gemm_ok<T>(r)) {
+        int rc = launch_real_gemm<T>(r, cp->ctx->stream);
+        if (rc) return rc;
+        continue;
+      }
+    }
     GemmArgs a = gemm_base<T>();
     a.M = cp->Nb[b]; a.N = cp->Nb[b] * w->nw; a.K = cp->Mb[b]; a.batch = 1;
     a.A = cp->phiT[b].p; a.lda = cp->Mb[b]; a.strideA = 0;
@@ -136,12 +214,28 @@ int gj_blocks(afqmc_cp cp, afqmc_walkers w, bool write_inverse, const int* alive
   return 0;
 }
 
-// X_b = W_b O_b^{-1} with green row-dot epilogue
+// X_b = W_b O_b^{-1} with green row-dot epilogue.  real: the imaginary parts of wf are zero and the
+// operators are real (real_ops), so everything here is.
 template <typename T>
-int green_gemm(afqmc_cp cp, afqmc_walkers w, DevBuf<char>* wf, const int* alive, bool kinetic) {
+int green_gemm(afqmc_cp cp, afqmc_walkers w, DevBuf<char>* wf, const int* alive, bool kinetic, int real = 0) {
   GroupFork fork;  // the blocks are independent: a grouped call launches them together
   for (int b = 0; b < cp->nblk; ++b) {
     fork.branch();
+    if (real && cp->Nb[b] <= WALKER_PANEL_NMAX) {
+      WalkerPanelArgs g;
+      memset(&g, 0, sizeof(g));
+      g.M = cp->Mb[b]; g.N = cp->Nb[b]; g.nw = w->nw;
+      g.W = wf[b].p; g.strideW = w->wsize(b);
+      g.B = cp->ovl[b].p; g.strideB = (long long)cp->Nb[b] * cp->Nb[b];
+      g.alive = alive;
+      g.P0 = cp->phiTr[b]; g.P2 = kinetic ? cp->wdkTr[b] : nullptr;
+      g.partner_half = cp->dense ? cp->L : 0;
+      g.out0 = cp->gpart[0][b].p; g.out1 = cp->dense ? cp->gpart[1][b].p : nullptr;
+      g.out2 = kinetic ? cp->gpart[2][b].p : nullptr;
+      int rc = launch_walker_green<T>(g, cp->ctx->stream);
+      if (rc) return rc;
+      continue;
+    }
     GemmArgs a = gemm_base<T>();
     a.M = cp->Mb[b]; a.N = cp->Nb[b]; a.K = cp->Nb[b]; a.batch = w->nw;
     a.A = wf[b].p; a.lda = cp->Mb[b]; a.strideA = w->wsize(b);
@@ -158,12 +252,28 @@ int green_gemm(afqmc_cp cp, afqmc_walkers w, DevBuf<char>* wf, const int* alive,
   return 0;
 }
 
-// W'_b = B_b diag(s) W_b  (all walkers, one GEMM per block)
+// W'_b = B_b diag(s) W_b  (all walkers, one GEMM per block).  real: the imaginary parts of the
+// input are zero (and, where scaled, those of the scale: real_ops).  A real B_b takes real products.
 template <typename T>
-int propagate_gemm(afqmc_cp cp, afqmc_walkers w, int which, DevBuf<char>* in, DevBuf<char>* out, bool scaled) {
+int propagate_gemm(afqmc_cp cp, afqmc_walkers w, int which, DevBuf<char>* in, DevBuf<char>* out, bool scaled,
+                   int real = 0) {
   GroupFork fork;  // the blocks are independent: a grouped call launches them together
   for (int b = 0; b < cp->nblk; ++b) {
     fork.branch();
+    if (cp->real_expk[which] && !(std::is_same<T, float>::value && cp->split_bf16)) {
+      RealGemmArgs r;
+      memset(&r, 0, sizeof(r));
+      r.M = cp->Mb[b]; r.N = cp->Nb[b] * w->nw; r.K = cp->Mb[b]; r.alpha = 1.0; r.b_real = real;
+      r.A = cp->expKr[which][b]; r.lda = cp->Mb[b];
+      r.B = in[b].p; r.ldb = cp->Mb[b];
+      r.C = out[b].p; r.ldc = cp->Mb[b];
+      if (scaled) { r.scale = cp->scale[b].p; r.scale_group = cp->Nb[b]; r.scale_strideG = cp->Mb[b]; }
+      if (real_gemm_ok<T>(r)) {
+        int rc = launch_real_gemm<T>(r, cp->ctx->stream);
+        if (rc) return rc;
+        continue;
+      }
+    }
     GemmArgs a = gemm_base<T>();
     a.M = cp->Mb[b]; a.N = cp->Nb[b] * w->nw; a.K = cp->Mb[b]; a.batch = 1;
     a.A = cp->expK[which][b].p; a.lda = cp->Mb[b];

@@ -412,6 +412,8 @@ int afqmc_capture_end(afqmc_ctx origin, afqmc_graph* out) {
     pairs.push_back({q.first, q.second, cs->first[i], swapped});
   }
   std::vector<afqmc_ctx> members = cs->members;
+  auto calls = std::move(cs->calls);
+  auto real_flags = std::move(cs->real_flags);
   delete cs;
   if (e != hipSuccess || e2 != hipSuccess || !g) {
     if (g) hipGraphDestroy(g);
@@ -423,6 +425,8 @@ int afqmc_capture_end(afqmc_ctx origin, afqmc_graph* out) {
   gr->origin = origin;
   gr->members = std::move(members);
   gr->pairs = std::move(pairs);
+  gr->calls = std::move(calls);
+  gr->real_flags = std::move(real_flags);
   e = hipGraphInstantiate(&gr->exec, g, nullptr, nullptr, 0);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&gr->ev, hipEventDisableTiming);
   if (e != hipSuccess) {
@@ -445,6 +449,28 @@ int afqmc_graph_launch(afqmc_graph g) {
   for (afqmc_ctx m : g->members) {
     HIP_TRY(hipEventRecord(g->ev, m->stream));
     HIP_TRY(hipStreamWaitEvent(s, g->ev, 0));
+  }
+  // captured for real walkers, and a set now holds complex ones: the calls themselves, in order,
+  // between the same fences as the graph
+  bool stale = false;
+  for (auto& f : g->real_flags) stale = stale || (f.second && !*f.first);
+  if (stale) {
+    if (!g->members.empty()) {
+      HIP_TRY(hipEventRecord(g->ev, s));
+      for (afqmc_ctx m : g->members) HIP_TRY(hipStreamWaitEvent(m->stream, g->ev, 0));
+    }
+    int rc = 0;
+    for (auto& call : g->calls)
+      if (!rc) rc = call();
+    for (afqmc_ctx m : g->members) {
+      HIP_TRY(hipEventRecord(g->ev, m->stream));
+      HIP_TRY(hipStreamWaitEvent(s, g->ev, 0));
+    }
+    if (!g->members.empty()) {
+      HIP_TRY(hipEventRecord(g->ev, s));
+      for (afqmc_ctx m : g->members) HIP_TRY(hipStreamWaitEvent(m->stream, g->ev, 0));
+    }
+    return rc;
   }
   // the graph reads each pair's data from the buffer it had at capture time: if eager calls
   // since then left the data in the other buffer, move it back first

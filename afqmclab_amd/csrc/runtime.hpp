@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <functional>
 #include <utility>
 #include <vector>
 
@@ -36,11 +37,24 @@ struct CaptureSession {
   std::vector<afqmc_ctx> members;
   std::vector<std::pair<DevBuf<char>*, DevBuf<char>*>> pairs;
   std::vector<void*> first;  // pairs[i].first->p when the pair was noted
+  // the recorded calls, and the walker sets' `real` flags (where they are and what they were): work
+  // captured for real walkers does not hold for a set that is later given complex ones, and a launch
+  // then makes the calls again instead
+  std::vector<std::function<int()>> calls;
+  std::vector<std::pair<const int*, int>> real_flags;
 };
 extern thread_local CaptureSession* g_capture;
 inline bool capturing() { return g_capture != nullptr; }
 inline hipError_t sync_unless_capturing(hipStream_t s) { return g_capture ? hipSuccess : hipStreamSynchronize(s); }
 void capture_note_pair(DevBuf<char>* a, DevBuf<char>* b);
+// notes the `real` flag a captured call relies on
+inline void capture_note_real(const int* real) {
+  if (g_capture) g_capture->real_flags.push_back({real, *real});
+}
+// records a call that has just been captured
+inline void capture_note_call(std::function<int()> call) {
+  if (g_capture) g_capture->calls.push_back(std::move(call));
+}
 #define NOT_CAPTURING() REQUIRE(!capturing(), "%s cannot be recorded into a graph (it synchronises)", __func__)
 
 struct GraphPair {
@@ -55,6 +69,8 @@ struct afqmc_graph_s {
   afqmc_ctx origin = nullptr;
   std::vector<afqmc_ctx> members;
   std::vector<GraphPair> pairs;
+  std::vector<std::function<int()>> calls;
+  std::vector<std::pair<const int*, int>> real_flags;
   hipEvent_t ev = nullptr;
 };
 

@@ -382,6 +382,15 @@ int afqmc_ph_adjust_ET(afqmc_ph ph);
 int afqmc_test_zgemm(afqmc_ctx ctx, int precision, int opa, int M, int N, int K, int batch, const double* A,
                      long long strideA, const double* B, const double* scale, int scale_group, int flags, int tile,
                      double* C);
+/* C = op(A) diag(scale) B with a real A (M x K, op_t: K x M) and complex B and C; b_real: the imaginary parts
+ * of B and scale are taken as zero */
+int afqmc_test_real_gemm(afqmc_ctx ctx, int precision, int op_t, int M, int N, int K, const double* A, const double* B,
+                         const double* scale, int scale_group, int b_real, double* C);
+/* per-walker products of real walkers (imaginary parts taken as zero, N <= 128): what = 1: out = W B (in place
+ * on the device, B upper triangular with b_upper; dead walkers keep W), 2: out = W^T W (zero for dead walkers);
+ * precision 1: FP32 walkers, FP64 products */
+int afqmc_test_walker_panel(afqmc_ctx ctx, int precision, int what, int M, int N, int nw, const double* W,
+                            const double* B, int b_upper, const int* alive, double* out);
 /* batched N x N inverse and log-determinant (Gauss-Jordan, partial pivoting), 1 <= N <= 256 */
 int afqmc_test_gj_inverse(afqmc_ctx ctx, int precision, int N, int batch, const double* A, double* Ainv,
                           double* logdet, int* info);

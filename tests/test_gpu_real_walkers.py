@@ -1,0 +1,176 @@
+"""Kernels for real operators and real walkers: the products against numpy, and whole calls on real
+walkers against the same walkers with a phase on one column (complex data, so the general kernels),
+whose overlaps, Green's functions, fields and energies are the same."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+from afqmclab_amd._lib import check, dptr, iptr, lib  # noqa: E402
+from afqmclab_amd.cp import CPMethod, CPPropagator  # noqa: E402
+from afqmclab_amd.model import HubbardModel, free_electron_trial, spin_block_trial  # noqa: E402
+from tests.gpu_util import crand, ctx  # noqa: E402
+
+EPS = {0: 2.0 ** -53, 1: 2.0 ** -24}
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("op_t", [0, 1])
+@pytest.mark.parametrize("b_real", [0, 1])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (16, 64, 16), (17, 65, 15), (37, 1200, 29), (112, 2100, 256),
+                                   (130, 1100, 33), (256, 9000, 48)])
+def test_real_gemm_matches_numpy(precision, op_t, b_real, shape):
+    """Every rounding of a K-term sum of products bounded by 1 is below K eps (two products per
+    complex element, so no cross terms)."""
+    M, N, K = shape
+    rng = np.random.default_rng(M + N + K + op_t)
+    A = rng.uniform(-1, 1, (M, K))
+    B = crand(rng, K, N)
+    group = 7
+    scale = None if op_t else crand(rng, (N + group - 1) // group, K)
+    C = np.zeros((N, M), dtype=np.complex128)
+    Abuf = np.ascontiguousarray(A if op_t else A.T)  # op T: K x M column-major
+    Bbuf = np.ascontiguousarray(B.T)
+    sbuf = None if scale is None else np.ascontiguousarray(scale)
+    check(lib().afqmc_test_real_gemm(ctx().h, precision, op_t, M, N, K, dptr(Abuf), dptr(Bbuf), dptr(sbuf), group,
+                                     b_real, dptr(C)))
+    S = 1.0 if scale is None else scale[np.arange(N) // group].T
+    if b_real:
+        B, S = B.real, np.real(S)
+    ref = A @ (S * B)
+    assert np.max(np.abs(C.T - ref)) <= 4 * (K + 4) * EPS[precision]
+    if b_real:
+        assert np.all(C.imag == 0)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("M,N", [(1, 1), (9, 3), (16, 16), (33, 17), (40, 31), (64, 48), (100, 63), (144, 65), (256, 112),
+                                 (300, 128)])
+def test_walker_products_match_numpy(precision, M, N):
+    """W B (general and upper triangular B, in place) and W^T W; FP32 walkers take FP64 products, so
+    only the stored result is rounded to FP32.  Dead walkers are left alone."""
+    rng = np.random.default_rng(M + N)
+    nw = 5
+    W = rng.uniform(-1, 1, (nw, M, N))
+    if precision:
+        W = W.astype(np.float32).astype(np.float64)
+    alive = np.array([1, 0, 1, 1, 1], dtype=np.int32)
+    Wbuf = np.ascontiguousarray(W.transpose(0, 2, 1)).astype(np.complex128)
+    for upper in (0, 1):
+        B = rng.uniform(-1, 1, (nw, N, N))
+        B = np.triu(B) if upper else B
+        Bbuf = np.ascontiguousarray(B.transpose(0, 2, 1)).astype(np.complex128)
+        out = np.zeros_like(Wbuf)
+        check(lib().afqmc_test_walker_panel(ctx().h, precision, 1, M, N, nw, dptr(Wbuf), dptr(Bbuf), upper, iptr(alive),
+                                            dptr(out)))
+        ref = np.where(alive[:, None, None] != 0, W @ B, W).transpose(0, 2, 1)
+        bound = 2 * (N + 2) * EPS[0] + (2 * N * EPS[1] if precision else 0.0)
+        assert np.max(np.abs(out - ref)) <= bound
+    out = np.zeros((nw, N, N), dtype=np.complex128)
+    check(lib().afqmc_test_walker_panel(ctx().h, precision, 2, M, N, nw, dptr(Wbuf), None, 0, iptr(alive), dptr(out)))
+    ref = np.where(alive[:, None, None] != 0, W.transpose(0, 2, 1) @ W, 0.0)
+    assert np.max(np.abs(out - ref)) <= 2 * (M + 2) * EPS[0]
+    assert np.array_equal(out, out.transpose(0, 2, 1))
+
+
+def pair(nx, ny, nup, ndn, dense, precision, nw=4, decomp="densitySpin", U=6.0, seed=3):
+    """Two propagators with real walkers and the same walkers with a phase on their first column."""
+    model = HubbardModel.square(nx, ny, nup + ndn, U)
+    L = model.L
+    phi = free_electron_trial(model) if dense else spin_block_trial(model, nup, ndn)
+    m = CPMethod(dt=0.02, decompType=decomp, walkerSizePerThread=nw)
+    rng = np.random.default_rng(seed)
+    wfs = []
+    for _ in range(nw):
+        w = np.zeros_like(phi)
+        noise = 0.3 / np.sqrt(L) * rng.uniform(-1, 1, phi.shape)
+        w[:] = phi + (noise if dense else np.where(phi_mask(L, nup, phi.shape), noise, 0.0))
+        wfs.append(w)
+    logw = 0.1 * rng.uniform(-1, 1, nw) + 0j
+    theta = 0.6
+    out = []
+    for phase in (0.0, theta):
+        prop = CPPropagator(ctx(), model, m, phi, nup=nup, spin_blocks=not dense, precision=precision, max_walkers=nw)
+        prop.set_seed(11)
+        prop.set_ET(-3.0)
+        ws = prop.walkers(nw)
+        up = [w.copy() for w in wfs]
+        for w in up:
+            w[:, 0] *= np.exp(1j * phase)
+        ws.upload(up, logw - 1j * phase)
+        out.append((prop, ws))
+    return out
+
+
+def phi_mask(L, nup, shape):
+    mask = np.zeros(shape, dtype=bool)
+    mask[:L, :nup] = mask[L:, nup:] = True
+    return mask
+
+
+def same(a, b, rtol):
+    a, b = np.asarray(a), np.asarray(b)
+    assert np.max(np.abs(a - b)) <= rtol * max(1e-300, np.max(np.abs(b))), np.max(np.abs(a - b)) / np.max(np.abs(b))
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("nx,ny,nup,ndn,dense", [(3, 3, 1, 2, False), (4, 4, 5, 7, False), (6, 6, 16, 15, False),
+                                                 (6, 6, 17, 18, False), (9, 7, 31, 28, False), (12, 12, 64, 65, False),
+                                                 (16, 16, 112, 97, False), (17, 16, 129, 128, False),
+                                                 (3, 3, 2, 2, True), (4, 4, 5, 5, True), (8, 8, 28, 29, True)])
+def test_real_walkers_equal_the_general_path(precision, nx, ny, nup, ndn, dense):
+    # 30 roundings' worth of FP64; FP32 overlaps of up to 129 electrons lose about 1e-5 in log det
+    rtol = 1e-10 if precision == 0 else 2e-3
+    (pr, wr), (pc, wc) = pair(nx, ny, nup, ndn, dense, precision)
+    same(np.exp(pr.log_overlap(wr)), np.exp(pc.log_overlap(wc)), rtol)
+    for a, b in zip(pr.green_diagonal(wr), pc.green_diagonal(wc)):
+        same(a + 1.0, b + 1.0, rtol)  # off-diagonal parts may be zero
+    for i in range(2):
+        (fr, xr), (fc, xc) = pr.step(wr, record=True), pc.step(wc, record=True)
+        on = wr.alive() != 0
+        assert np.array_equal(on, wc.alive() != 0) and on.any()
+        assert np.array_equal(xr[on], xc[on])
+        assert np.max(np.abs(fr[on] - fc[on])) <= rtol
+        pr.stabilize(wr)
+        pc.stabilize(wc)
+    for p, w in ((pr, wr), (pc, wc)):
+        p.onebody(w, 1)
+        p.measure(w)
+    er, ec = pr.energy(), pc.energy()
+    same([er[k] for k in ("den", "HNum", "KNum", "VNum")], [ec[k] for k in ("den", "HNum", "KNum", "VNum")], rtol)
+    same(pr.site_measure(), pc.site_measure(), rtol)
+    wt, tb, _ = pr.pop_control(wr, record=True)
+    wt2, tb2, _ = pc.pop_control(wc, record=True)
+    same(wt, wt2, rtol)
+    wf, _, _ = wr.download()
+    assert np.all(wf.imag == 0)
+
+
+def test_graph_of_real_walkers_serves_complex_ones():
+    """A graph captured while the walkers are real, launched after complex walkers were uploaded,
+    gives what the calls themselves give, and real walkers uploaded later take the graph again."""
+    (pr, wr), (pc, wc) = pair(4, 4, 5, 5, False, 0)
+    real, _, _ = wr.download()
+    c, _, _ = wc.download()
+    ctx().capture_begin()
+    pr.step(wr)
+    pr.stabilize(wr)
+    pr.measure(wr)
+    g = ctx().capture_end()
+    for k, w in enumerate((real, c, real, c)):
+        wr.upload(w)
+        wc.upload(w)
+        for p in (pr, pc):
+            p.reset_measure()
+            p.set_seed(5 + k)
+        for _ in range(3):
+            g.launch()
+            pc.step(wc)
+            pc.stabilize(wc)
+            pc.measure(wc)
+            ctx().synchronize()
+        a, b = wr.download(), wc.download()
+        same(a[0], b[0], 1e-12)
+        same(a[1] + 1.0, b[1] + 1.0, 1e-12)
+        same(list(pr.energy().values()), list(pc.energy().values()), 1e-11)
+    g.close()
