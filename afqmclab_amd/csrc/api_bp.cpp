@@ -137,7 +137,7 @@ int measure_impl(afqmc_bp bp, afqmc_walkers w, int snap_slot) {
     a.alive = w->alive.p;
     if ((rc = launch_cgemm<T>(OP_C, EPI_STORE, a, s))) return rc;
   }
-  if ((rc = gj_blocks<T>(cp, w, true, w->alive.p))) return rc;
+  if ((rc = gj_blocks<T>(cp, w, true, w->alive.p, bra->real && ket->real))) return rc;
   for (int b = 0; b < cp->nblk; ++b) {
     const int Mb = cp->Mb[b], Nb = cp->Nb[b];
     GemmArgs a = gemm_base<T>();

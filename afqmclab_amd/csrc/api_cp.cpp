@@ -78,7 +78,7 @@ LogOArgs logo_args(afqmc_cp cp, afqmc_walkers w, int mode) {
 template <typename T>
 int do_overlap(afqmc_cp cp, afqmc_walkers w, bool inverse) {
   int rc = overlap_gemm<T>(cp, w, w->wf, w->real);
-  if (!rc) rc = gj_blocks<T>(cp, w, inverse, w->alive.p);
+  if (!rc) rc = gj_blocks<T>(cp, w, inverse, w->alive.p, w->real);
   return rc;
 }
 
@@ -115,7 +115,7 @@ int step_impl(afqmc_cp cp, afqmc_walkers w, double* force_out, int* aux_out, int
   }
   {
     RegionTimer t(cp->ctx, REG_GJ);
-    if ((rc = gj_blocks<T>(cp, w, true, w->alive.p))) return rc;
+    if ((rc = gj_blocks<T>(cp, w, true, w->alive.p, w->real))) return rc;
   }
   LogOArgs l = logo_args<T>(cp, w, LOGO_STEP);
   if ((rc = launch_logo(l, s))) return rc;
@@ -275,7 +275,7 @@ int measure_impl(afqmc_cp cp, afqmc_walkers w) {
   if ((rc = propagate_gemm<T>(cp, w, 2, w->wf, w->tmp, false, w->real))) return rc;
   if ((rc = launch_logw_shift(w->nw, w->logw.p, w->logw_tmp.p, cp->hop_logw[2], s))) return rc;
   if ((rc = overlap_gemm<T>(cp, w, w->tmp, w->real))) return rc;
-  if ((rc = gj_blocks<T>(cp, w, true, w->alive.p))) return rc;
+  if ((rc = gj_blocks<T>(cp, w, true, w->alive.p, w->real))) return rc;
   LogOArgs l = logo_args<T>(cp, w, LOGO_MEASURE);
   l.logw = w->logw_tmp.p;
   if ((rc = launch_logo(l, s))) return rc;
@@ -301,7 +301,7 @@ int mixed_weight_impl(afqmc_cp cp, afqmc_walkers w) {
   if ((rc = propagate_gemm<T>(cp, w, 2, w->wf, w->tmp, false, w->real))) return rc;
   if ((rc = launch_logw_shift(w->nw, w->logw.p, w->logw_tmp.p, cp->hop_logw[2], s))) return rc;
   if ((rc = overlap_gemm<T>(cp, w, w->tmp, w->real))) return rc;
-  if ((rc = gj_blocks<T>(cp, w, false, w->alive.p))) return rc;
+  if ((rc = gj_blocks<T>(cp, w, false, w->alive.p, w->real))) return rc;
   LogOArgs l = logo_args<T>(cp, w, LOGO_MEASURE);
   l.logw = w->logw_tmp.p;
   return launch_logo(l, s);

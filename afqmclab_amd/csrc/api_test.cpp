@@ -100,7 +100,7 @@ int gj_t(afqmc_ctx ctx, int kind, int N, int batch, const double* A, double* Ain
   memset(&a, 0, sizeof(a));
   a.N = N; a.batch = batch; a.in = d.p; a.ld_in = N; a.stride_in = (long long)N * N;
   a.out = d.p; a.ld_out = N; a.stride_out = a.stride_in; a.logdet = ld.p; a.info = inf.p;
-  a.write_inverse = 1; a.nsub = N; a.alive_div = 1; a.layout = layout; a.alive = alive ? al.p : nullptr;
+  a.write_inverse = 1; a.nsub = N; a.alive_div = 1; a.layout = layout & 15; a.real = layout >> 4; a.alive = alive ? al.p : nullptr;
   a.work = wk.p;
   rc = kind == 0 ? launch_gj_inverse<T>(a, s) : launch_chol_inverse<T>(a, s);
   if (rc) return rc;
@@ -279,6 +279,13 @@ int afqmc_test_chol_inverse(afqmc_ctx ctx, int N, int batch, const double* S, do
   REQUIRE(ctx && S && Rinv && logsum, "null argument");
   ScopedDevice sd(ctx);
   return gj_t<double>(ctx, 1, N, batch, S, Rinv, logsum, info);
+}
+
+int afqmc_test_chol_inverse_real(afqmc_ctx ctx, int N, int batch, const double* S, double* Rinv, double* logsum,
+                                 int* info) {
+  REQUIRE(ctx && S && Rinv && logsum, "null argument");
+  ScopedDevice sd(ctx);
+  return gj_t<double>(ctx, 1, N, batch, S, Rinv, logsum, info, 16);
 }
 
 }  // extern "C"

@@ -195,8 +195,9 @@ int overlap_gemm(afqmc_cp cp, afqmc_walkers w, DevBuf<char>* wf, int real = 0) {
   return 0;
 }
 
+// (real: the imaginary parts of the overlaps are zero)
 template <typename T>
-int gj_blocks(afqmc_cp cp, afqmc_walkers w, bool write_inverse, const int* alive) {
+int gj_blocks(afqmc_cp cp, afqmc_walkers w, bool write_inverse, const int* alive, int real = 0) {
   GroupFork fork;  // the blocks are independent: a grouped call launches them together
   for (int b = 0; b < cp->nblk; ++b) {
     fork.branch();
@@ -208,6 +209,7 @@ int gj_blocks(afqmc_cp cp, afqmc_walkers w, bool write_inverse, const int* alive
     s.logdet = cp->ldet[b].p; s.info = cp->info[b].p; s.write_inverse = write_inverse ? 1 : 0;
     s.alive = alive; s.alive_div = 1;
     s.work = cp->gjwork[b].p;
+    s.real = real;
     int rc = launch_gj_inverse<T>(s, cp->ctx->stream);
     if (rc) return rc;
   }

@@ -397,7 +397,8 @@ int afqmc_test_gj_inverse(afqmc_ctx ctx, int precision, int N, int batch, const 
 /* the same with the kernel chosen: 1 lanes = rows (readlanes for the pivot row), 2 a 2-D lane layout
  * with both update operands from LDS (N <= 128), identical to 1; 3 panels of four columns with rank-4
  * updates (N <= 112), equal to 1 up to rounding (same pivots, updates summed in another order);
- * 0 the default for N and batch */
+ * 0 the default for N and batch; 16: the imaginary parts of A
+ * are taken as zero (real arithmetic, the default kernel for N) */
 int afqmc_test_gj_inverse_layout(afqmc_ctx ctx, int precision, int N, int batch, int layout, const double* A,
                                  double* Ainv, double* logdet, int* info);
 /* the same over the matrices b with alive[b] != 0 only; the others keep A (the inverse is written
@@ -410,6 +411,9 @@ int afqmc_test_copy(afqmc_ctx ctx, long long bytes, int reps, double* ms);
 /* batched Cholesky S = R^H R, returns R^{-1} and (sum log R_kk, same) */
 int afqmc_test_chol_inverse(afqmc_ctx ctx, int N, int batch, const double* S, double* Rinv, double* logsum,
                             int* info);
+/* the same with the imaginary parts of S taken as zero (real arithmetic) */
+int afqmc_test_chol_inverse_real(afqmc_ctx ctx, int N, int batch, const double* S, double* Rinv, double* logsum,
+                                 int* info);
 
 #ifdef __cplusplus
 }

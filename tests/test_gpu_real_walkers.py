@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 from afqmclab_amd._lib import check, dptr, iptr, lib  # noqa: E402
 from afqmclab_amd.cp import CPMethod, CPPropagator  # noqa: E402
 from afqmclab_amd.model import HubbardModel, free_electron_trial, spin_block_trial  # noqa: E402
-from tests.gpu_util import crand, ctx  # noqa: E402
+from tests.gpu_util import crand, ctx, gj_inverse_masked  # noqa: E402
 
 EPS = {0: 2.0 ** -53, 1: 2.0 ** -24}
 
@@ -174,3 +174,50 @@ def test_graph_of_real_walkers_serves_complex_ones():
         same(a[1] + 1.0, b[1] + 1.0, 1e-12)
         same(list(pr.energy().values()), list(pc.energy().values()), 1e-11)
     g.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("N", [1, 2, 4, 5, 15, 16, 17, 32, 33, 48, 49, 63, 64, 65, 80, 81, 97, 112, 113, 128, 129, 160])
+def test_gj_real_matches_lapack(precision, N):
+    """Inverse and log-determinant of real matrices in every size class, with a permutation, a singular matrix and a badly scaled one among them.  A backward-stable inverse is
+    within cond * N eps of the exact one; FP32 storage rounds the input-independent result once."""
+    rng = np.random.default_rng(N)
+    A = rng.standard_normal((6, N, N))
+    A[1] = np.eye(N)[rng.permutation(N)]
+    A[2] *= 1e-30 if precision else 1e-140
+    A[3] = A[3] @ np.diag(np.logspace(0, -6, N))
+    if precision:
+        A = A.astype(np.float32).astype(np.float64)
+    A[4][:, -1] = 0.0
+    alive = np.array([1, 1, 1, 1, 1, 0], dtype=np.int32)
+    Ainv, ld, info = gj_inverse_masked(A, alive, 16, precision, fill=7.0)
+    assert list(info[:5]) == [0, 0, 0, 0, 1]
+    assert np.array_equal(Ainv[5], A[5]) and ld[5] == 7.0
+    for b in range(4):
+        ref = np.linalg.inv(A[b])
+        cond = np.linalg.cond(A[b], 2)
+        bound = 8 * N * cond * EPS[0] + (2 * EPS[1] if precision else 0.0)
+        assert np.max(np.abs(Ainv[b] - ref)) <= bound * np.max(np.abs(ref))
+        assert np.all(Ainv[b].imag == 0)
+        sign, logabs = np.linalg.slogdet(A[b])
+        assert abs(ld[b].real - logabs) <= 8 * N * cond * EPS[0] * max(1.0, abs(logabs))
+        assert abs(np.exp(1j * ld[b].imag) - sign) < 1e-12
+
+
+@pytest.mark.parametrize("N", [1, 3, 16, 17, 33, 64, 65, 97, 112, 113, 128, 129, 160])
+def test_chol_real_matches_lapack(N):
+    rng = np.random.default_rng(N)
+    W = rng.standard_normal((4, N + 20, N))
+    S = np.ascontiguousarray(W.transpose(0, 2, 1) @ W).astype(np.complex128)
+    out, ld, info = np.zeros_like(S), np.zeros(4, dtype=np.complex128), np.zeros(4, dtype=np.int32)
+    S[3] -= 1.01 * np.linalg.eigvalsh(S[3])[-1] * np.eye(N)  # not positive definite
+    check(lib().afqmc_test_chol_inverse_real(ctx().h, N, 4, dptr(S), dptr(out), dptr(ld), iptr(info)))
+    assert list(info) == [0, 0, 0, 1]
+    for b in range(3):
+        R = np.linalg.cholesky(S[b].real).T
+        ref = np.linalg.inv(R)
+        cond = np.linalg.cond(S[b].real)
+        got = out[b].T  # column-major
+        assert np.max(np.abs(got - ref)) <= 8 * N * cond * EPS[0] * np.max(np.abs(ref))
+        assert np.all(np.tril(got, -1) == 0) and np.all(got.imag == 0)
+        assert abs(ld[b].real - np.sum(np.log(np.diag(R)))) <= 8 * N * cond * EPS[0]
