@@ -165,6 +165,7 @@ CholQrBlock qr_block(afqmc_cp cp, afqmc_walkers w, DevBuf<char>* wf, DevBuf<char
   q.info = cp->qrinfo[b].p; q.need = cp->qr_need.p; q.flag = cp->qr_flag.p;
   q.alive = w->alive.p; q.logw = w->logw.p;
   q.m0 = 1.0; q.m1 = 0.0; q.tol = tol; q.sc = cp->sc.p;
+  q.real = w->real != 0;
   return q;
 }
 
@@ -183,9 +184,18 @@ int stabilize_impl(afqmc_cp cp, afqmc_walkers w) {
     capture_note_pair(&cp->qr64[b], &cp->qr64b[b]);
   }
   if (!cp->fp32) return qr_impl_f64(cp, w, w->wf, w->tmp, 1e-13);
-  // mixed path: QR in FP64 on a widened copy of the FP32 walkers
   hipStream_t s = cp->ctx->stream;
   int rc;
+  if (w->real && cp->Nb[0] <= WALKER_PANEL_NMAX && cp->Nb[1] <= WALKER_PANEL_NMAX) {
+    // real walkers: no FP64 copies (the overlap buffer takes the check's Gram matrices)
+    for (int b = 0; b < cp->nblk; ++b) {
+      const CholQrBlock q = qr_block(cp, w, cp->qr64, cp->qr64b, b, 1e-8);
+      if ((rc = cholqr_real_f32(q, w->wf[b].p, w->tmp[b].p, cp->ovl[b].p, cp->qr_mask.p, 1e-4, s))) return rc;
+      std::swap(w->wf[b], w->tmp[b]);
+    }
+    return 0;
+  }
+  // mixed path: QR in FP64 on a widened copy of the FP32 walkers
   {
     GroupFork fork;
     for (int b = 0; b < cp->nblk; ++b) {
@@ -507,6 +517,7 @@ int afqmc_cp_create(afqmc_ctx ctx, const afqmc_cp_desc* d, afqmc_cp* out) {
   if (!rc) rc = cp->comb_num.alloc(nw);
   if (!rc) rc = cp->qr_need.alloc(nw);
   if (!rc) rc = cp->qr_flag.alloc(nw);
+  if (!rc) rc = cp->qr_mask.alloc(nw);
   if (!rc) rc = cp->comb_prob.alloc(nw);
   if (!rc) rc = cp->weight.alloc(nw);
   if (!rc) rc = cp->per_walker.alloc((size_t)nw * 8);

@@ -4,6 +4,7 @@
 #pragma once
 #include "cp_kernels.hpp"
 #include "runtime.hpp"
+#include "walker_panel.hpp"
 
 struct CholQrBlock {
   int nw = 0, M = 0, N = 0, nsub = 0;   // walkers, rows, columns; nsub: columns of the second log sum
@@ -18,6 +19,9 @@ struct CholQrBlock {
   double tol = 1e-13;                   // second pass where |Q^H Q - I| exceeds this
   DevScalars* sc = nullptr;             // counts of shifted and dead walkers
   bool check_all = true;                // pass 2 over every alive walker (else the caller's own check)
+  // every imaginary part of the walkers is zero: real products and factorisations (up to
+  // WALKER_PANEL_NMAX columns; wider walkers take the general kernels, which keep them zero)
+  bool real = false;
 };
 
 // W <- Q with W = Q R, R upper triangular with positive diagonal; logw += log det R (by m0, m1).
@@ -36,6 +40,14 @@ struct CholQrBlock {
 // With check_all false pass 2 is left to the caller, which runs cholqr_refine over the walkers its
 // own check selects.
 int cholqr_f64(const CholQrBlock& q, hipStream_t s);
+// The same for real FP32 walkers (real set, N <= WALKER_PANEL_NMAX), without FP64 copies of the walkers: the
+// Gram matrix is formed in FP64 from the FP32 walkers, and W R^-1 in FP64 is rounded once, into `out`
+// (another buffer of the walkers' size; w32 keeps W).  Only the walkers that need the shifted pass or
+// a further one (their FP32 result farther than check_tol from orthonormal, by an FP32 Gram matrix
+// in gram32, [nw][N][N] complex FP32) are widened: q.wf, q.tmp are FP64 buffers used for those.
+// mask: [nw] workspace.
+int cholqr_real_f32(const CholQrBlock& q, const void* w32, void* out, void* gram32, int* mask, double check_tol,
+                    hipStream_t s);
 // A further CholeskyQR of the walkers in `among` whose Q^H Q is farther than tol from I (need
 // lists them afterwards); the others stay put.
 int cholqr_refine(const CholQrBlock& q, const int* among, hipStream_t s);

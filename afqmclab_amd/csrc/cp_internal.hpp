@@ -46,7 +46,7 @@ struct afqmc_cp_s {
   DevBuf<char> ovl[2], scale[2], d2x2, qrS[2], qr64[2], qr64b[2];
   DevBuf<char> gjwork[2];  // FP64 working copies of the overlap matrices above 160 columns
   DevBuf<zd> ldet[2], qrld[2], logO, gpart[3][2], per_walker, site_acc, site_part, den;
-  DevBuf<int> info[2], qrinfo[2], prefix, table, comb_num, qr_need, qr_flag;
+  DevBuf<int> info[2], qrinfo[2], prefix, table, comb_num, qr_need, qr_flag, qr_mask;
   DevBuf<double> weight, comb_prob, force_rec;
   DevBuf<int> aux_rec, aux_in;
   int ntile[2] = {1, 1};

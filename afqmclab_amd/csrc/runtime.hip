@@ -135,6 +135,7 @@ struct ConvertMaskedArgs {
   cplx<B>* out;
   const int* mask;
   long long n;
+  int nw;
 };
 template <typename A, typename B>
 struct ConvertMaskedK {
@@ -143,13 +144,21 @@ struct ConvertMaskedK {
 };
 template <typename A, typename B>
 __device__ __forceinline__ void ConvertMaskedK<A, B>::run(const BlockIdx3& bk, const ConvertMaskedArgs<A, B>& g) {
-  const int w = bk.y;
-  if (!g.mask[w]) return;
   const long long n = g.n;
-  const cplx<A>* in = g.in + (long long)w * n;
-  cplx<B>* out = g.out + (long long)w * n;
-  for (long long i = (long long)bk.x * blockDim.x + threadIdx.x; i < n; i += (long long)bk.gx * blockDim.x)
-    out[i] = cmk<B>((B)in[i].re, (B)in[i].im);
+  for (int w = bk.y; w < g.nw; w += bk.gy) {
+    if (!g.mask[w]) continue;
+    const cplx<A>* in = g.in + (long long)w * n;
+    cplx<B>* out = g.out + (long long)w * n;
+    for (long long i = (long long)bk.x * blockDim.x + threadIdx.x; i < n; i += (long long)bk.gx * blockDim.x)
+      out[i] = cmk<B>((B)in[i].re, (B)in[i].im);
+  }
+}
+// Copies masked by walker: up to 64 workgroups across a walker's elements, about 4096 in all, each
+// looping over walkers.  A mask that is usually empty (the QR's further passes) then costs a few
+// microseconds where one workgroup per 256 elements and walker cost 28 to 49 for 2048 walkers.
+dim3 masked_grid(long long per_walker, int nw) {
+  const unsigned gx = (unsigned)std::min<long long>((per_walker + 255) / 256, 64);
+  return dim3(gx, (unsigned)std::min(nw, std::max(1, 4096 / (int)gx)));
 }
 
 __global__ void logw_shift_kernel(int nw, const zd* logw, zd* out, zd c) {
@@ -170,6 +179,7 @@ struct SelectArgs {
   const E* src;
   E* dst;
   long long n;
+  int nw;
 };
 template <typename E>
 struct SelectK {
@@ -179,10 +189,11 @@ struct SelectK {
 template <typename E>
 __device__ __forceinline__ void SelectK<E>::run(const BlockIdx3& bk, const SelectArgs<E>& g) {
   const long long n = g.n;
-  const int w = bk.y;
-  if (!g.alive[w]) return;
-  for (long long i = (long long)bk.x * blockDim.x + threadIdx.x; i < n; i += (long long)bk.gx * blockDim.x)
-    g.dst[(long long)w * n + i] = g.src[(long long)w * n + i];
+  for (int w = bk.y; w < g.nw; w += bk.gy) {
+    if (!g.alive[w]) continue;
+    for (long long i = (long long)bk.x * blockDim.x + threadIdx.x; i < n; i += (long long)bk.gx * blockDim.x)
+      g.dst[(long long)w * n + i] = g.src[(long long)w * n + i];
+  }
 }
 __global__ void reset_measure_kernel(DevScalars* sc, zd* site_acc, int L) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -211,9 +222,14 @@ int launch_convert_f64_f32(const void* in, void* out, long long n, hipStream_t s
 int launch_convert_f64_f32_masked(const void* in, void* out, long long per_walker, int nw, const int* mask,
                                   hipStream_t s) {
   if (nw <= 0 || per_walker <= 0) return 0;
-  ConvertMaskedArgs<double, float> a{(const zd*)in, (zf*)out, mask, per_walker};
-  const unsigned gx = (unsigned)std::min<long long>((per_walker + 255) / 256, 64);
-  return glaunch<ConvertMaskedK<double, float>>(a, dim3(gx, nw), dim3(256), 0, s);
+  ConvertMaskedArgs<double, float> a{(const zd*)in, (zf*)out, mask, per_walker, nw};
+  return glaunch<ConvertMaskedK<double, float>>(a, masked_grid(per_walker, nw), dim3(256), 0, s);
+}
+int launch_convert_f32_f64_masked(const void* in, void* out, long long per_walker, int nw, const int* mask,
+                                  hipStream_t s) {
+  if (nw <= 0 || per_walker <= 0) return 0;
+  ConvertMaskedArgs<float, double> a{(const zf*)in, (zd*)out, mask, per_walker, nw};
+  return glaunch<ConvertMaskedK<float, double>>(a, masked_grid(per_walker, nw), dim3(256), 0, s);
 }
 int launch_logw_shift(int nw, const zd* logw, zd* out, zd c, hipStream_t s) {
   hipLaunchKernelGGL(logw_shift_kernel, dim3((nw + 255) / 256), dim3(256), 0, s, nw, logw, out, c);
@@ -232,12 +248,12 @@ int launch_logw_vec_add(int nw, zd* logw, const int* alive, const zd* v, hipStre
 }
 int launch_select_alive(int nw, long long n, size_t esz, const int* alive, const void* src, void* dst, hipStream_t s) {
   if (nw <= 0 || n <= 0) return 0;
-  dim3 grid((unsigned)std::min<long long>((n + 255) / 256, 1024), nw);
+  const dim3 grid = masked_grid(n, nw);
   if (esz == 16) {
-    SelectArgs<uint4> g{alive, (const uint4*)src, (uint4*)dst, n};
+    SelectArgs<uint4> g{alive, (const uint4*)src, (uint4*)dst, n, nw};
     return glaunch<SelectK<uint4>>(g, grid, dim3(256), 0, s);
   }
-  SelectArgs<uint2> g{alive, (const uint2*)src, (uint2*)dst, n};
+  SelectArgs<uint2> g{alive, (const uint2*)src, (uint2*)dst, n, nw};
   return glaunch<SelectK<uint2>>(g, grid, dim3(256), 0, s);
 }
 int launch_reset_measure(DevScalars* sc, zd* site_acc, int L, hipStream_t s) {

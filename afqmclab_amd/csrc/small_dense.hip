@@ -288,7 +288,7 @@ int dispatch(int kind, const SmallDenseArgs& a, hipStream_t s) {
     return glaunch<CholWideK>(a, dim3(a.batch), dim3(64 * WAVES), 0, s);
   }
   if (a.real) return small_dense_real<T>(kind, a, s);
-  return dispatch_registers<T, zd>(kind, a, s);
+  return small_dense_complex<T>(kind, a, s);
 }
 
 }  // namespace

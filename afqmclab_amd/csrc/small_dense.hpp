@@ -24,7 +24,10 @@ long long small_dense_gj_work_bytes(int N, int batch);
 
 template <typename T> int launch_gj_inverse(const SmallDenseArgs& a, hipStream_t s);
 template <typename T> int launch_chol_inverse(const SmallDenseArgs& a, hipStream_t s);
-// the register kernels (N <= 160) on real matrices; kind 0: Gauss-Jordan, 1: Cholesky
+// the register kernels (N <= 160) on complex and on real matrices; kind 0: Gauss-Jordan, 1: Cholesky
+template <typename T> int small_dense_complex(int kind, const SmallDenseArgs& a, hipStream_t s);
+template <> int small_dense_complex<double>(int kind, const SmallDenseArgs& a, hipStream_t s);
+template <> int small_dense_complex<float>(int kind, const SmallDenseArgs& a, hipStream_t s);
 template <typename T> int small_dense_real(int kind, const SmallDenseArgs& a, hipStream_t s);
 template <> int small_dense_real<double>(int kind, const SmallDenseArgs& a, hipStream_t s);
 template <> int small_dense_real<float>(int kind, const SmallDenseArgs& a, hipStream_t s);

@@ -1,6 +1,6 @@
 // The register-resident small dense kernels and their dispatch, for complex (E = zd) and real
-// (E = double) working matrices; each is compiled in a file of its own (small_dense.hip,
-// small_dense_real.hip).
+// (E = double) working matrices; each combination with a storage type is compiled in a file of its
+// own (small_dense_complex_*.hip, small_dense_real_*.hip).
 #pragma once
 #include "small_dense.hpp"
 

@@ -221,3 +221,49 @@ def test_chol_real_matches_lapack(N):
         assert np.max(np.abs(got - ref)) <= 8 * N * cond * EPS[0] * np.max(np.abs(ref))
         assert np.all(np.tril(got, -1) == 0) and np.all(got.imag == 0)
         assert abs(ld[b].real - np.sum(np.log(np.diag(R)))) <= 8 * N * cond * EPS[0]
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("nx,ny,nup,ndn", [(4, 4, 1, 5), (6, 6, 16, 17), (8, 8, 33, 31), (12, 12, 64, 65), (16, 16, 112, 128)])
+def test_qr_of_ill_conditioned_real_walkers(precision, nx, ny, nup, ndn):
+    """Orthonormal result, log det R and the span for well- and ill-conditioned walkers (nearly
+    parallel columns, which take the shifted pass); a walker with two equal columns dies."""
+    model = HubbardModel.square(nx, ny, nup + ndn, 4.0)
+    L, nw = model.L, 6
+    phi = spin_block_trial(model, nup, ndn)
+    m = CPMethod(dt=0.02, walkerSizePerThread=nw)
+    prop = CPPropagator(ctx(), model, m, phi, nup=nup, spin_blocks=True, precision=precision, max_walkers=nw)
+    rng = np.random.default_rng(nup)
+    wfs = []
+    for k in range(nw):
+        w = np.where(phi_mask(L, nup, phi.shape), rng.uniform(-1, 1, phi.shape), 0.0) + 0j
+        if k == 2:  # condition about 1e6
+            w[L:, -1] = w[L:, -2] + 1e-6 * w[L:, -1]
+        if k == 3:
+            w[L:, -1] = w[L:, -2]
+        if k == 4:
+            w *= 1e4
+        wfs.append(w if precision == 0 else w.astype(np.complex64).astype(np.complex128))
+    ws = prop.walkers(nw)
+    ws.upload(wfs, np.zeros(nw))
+    prop.stabilize(ws)
+    q, lw, alive = ws.download()
+    eps = 1e-12 if precision == 0 else 4e-6
+    assert list(alive[[0, 1, 2, 4, 5]]) == [1, 1, 1, 1, 1]
+    # equal columns: dead, or (a last rounding apart) a log-weight that weighs nothing
+    assert alive[3] == 0 or lw[3].real < lw[0].real - 20
+    shifted, killed = prop.qr_stats()
+    assert shifted >= 1 and killed == 1 - alive[3]
+    for k in (0, 1, 2, 4, 5):
+        Q = q[k]
+        assert np.max(np.abs(Q.conj().T @ Q - np.eye(nup + ndn))) < eps
+        R = np.linalg.qr(wfs[k])[1]
+        # log det R: u kappa^2 of an unshifted Cholesky (kappa <= 1e3 here), and u kappa c with the
+        # shift's c = 11 (M N + N^2) <= 1e6 for the walker with kappa = 1e6
+        ref = np.sum(np.log(np.abs(np.diag(R))))
+        assert abs(lw[k].real - ref) < (1e-4 if k == 2 else 1e-9) * max(1.0, abs(ref))
+        R = Q.conj().T @ wfs[k]  # upper triangular with a positive diagonal: Q spans W
+        size = np.max(np.abs(R))
+        assert np.max(np.abs(np.tril(R, -1))) < 20 * eps * size
+        assert np.all(np.diag(R).real > 0)
+        assert np.max(np.abs(Q @ R - wfs[k])) < 20 * eps * size
