@@ -14,7 +14,9 @@
 #include "../../include/afqmc_mi355x.h"
 #include "cp_kernels.hpp"
 #include "gemm.hpp"
+#include "ph_exchange.hpp"
 #include "ph_kernels.hpp"
+#include "real_gemm.hpp"
 #include "runtime.hpp"
 #include "small_dense.hpp"
 
@@ -36,6 +38,17 @@ __global__ void transpose_half_rot(int L, int Ns, int G, const cplx<double>* in,
     out[e] = from_zd<T>(in[j + (long long)i * Ns + g * (long long)Ns * L]);
   }
 }
+// the same of real vectors: real output
+template <typename T>
+__global__ void transpose_half_rot_real(int L, int Ns, int G, const double* in, T* out) {
+  const long long tot = (long long)L * Ns * G;
+  for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < tot; e += (long long)gridDim.x * blockDim.x) {
+    const long long g = e / ((long long)L * Ns);
+    const long long r = e - g * L * Ns;
+    const int i = (int)(r % L), j = (int)(r / L);
+    out[e] = (T)in[2 * (j + (long long)i * Ns + g * (long long)Ns * L)];
+  }
+}
 }  // namespace
 
 struct afqmc_ph_s {
@@ -47,6 +60,7 @@ struct afqmc_ph_s {
   zd sqrt_minus_dt{0, 0};
   zd trial_logw{0, 0};
   DevBuf<char> phiT[2], wdtT[2], Lvec, Ahalf[2], onebody[3];
+  int real_half = 0;  // the half-rotated vectors of both spins have no imaginary part: Ahalf holds real numbers
   int onebody_log[3] = {0, 0, 0};
   zd onebody_logw[3];
   int ob_set[3] = {0, 0, 0};
@@ -77,6 +91,14 @@ struct afqmc_ph_walkers_s {
 };
 
 namespace {
+
+// real half-rotated vectors with both spins within the fused kernel's range: exchange and background
+// of a measurement come from its traces, without the blocks D in memory
+bool ph_traces(afqmc_ph ph) {
+  for (int sp = 0; sp < 2; ++sp)
+    if (!(ph->fp32 ? ph_exchange_ok<float>(ph->L, ph->Ns[sp]) : ph_exchange_ok<double>(ph->L, ph->Ns[sp]))) return false;
+  return ph->real_half != 0;
+}
 
 GemmArgs gbase() {
   GemmArgs a;
@@ -134,6 +156,18 @@ template <typename T>
 int ph_background(afqmc_ph ph, afqmc_ph_walkers w) {
   for (int sp = 0; sp < 2; ++sp) {
     const long long K = (long long)ph->L * ph->Ns[sp];
+    if (ph->real_half) {  // 0.73 ms a spin at G = 1600, 1024 walkers and K = 8000, 1.00 as complex products
+      RealGemmArgs r;
+      memset(&r, 0, sizeof(r));
+      r.M = ph->G; r.N = w->nw; r.K = (int)K; r.op_t = 1;
+      r.A = ph->Ahalf[sp].p; r.lda = K;
+      r.B = ph->X[sp].p; r.ldb = K;
+      r.C = ph->bgbuf.p; r.ldc = ph->G;
+      r.alpha = 1.0; r.beta_one = sp;
+      int rc = launch_real_gemm<T>(r, ph->ctx->stream);
+      if (rc) return rc;
+      continue;
+    }
     GemmArgs a = gbase();
     a.M = ph->G; a.N = w->nw; a.K = (int)K; a.batch = 1;
     a.A = ph->Ahalf[sp].p; a.lda = K;
@@ -378,7 +412,8 @@ int ph_measure_impl(afqmc_ph ph, afqmc_ph_walkers w) {
   LogOArgs l = ph_logo_args(ph, w, LOGO_MEASURE, w->logw_tmp.p);
   if ((rc = launch_logo(l, s))) return rc;
   if ((rc = ph_theta<T>(ph, w, tmpw, w->alive.p))) return rc;
-  if ((rc = ph_background<T>(ph, w))) return rc;
+  const bool traces = ph_traces(ph);
+  if (!traces && (rc = ph_background<T>(ph, w))) return rc;
   // kinetic: sum_s sum_ij X_s(i,j) (phiT_s^H t)^T(i,j)
   for (int sp = 0; sp < 2; ++sp) {
     const long long n = (long long)ph->L * ph->Ns[sp];
@@ -391,8 +426,28 @@ int ph_measure_impl(afqmc_ph ph, afqmc_ph_walkers w) {
   // side by side as B (N = Ns * chunk), A panels reused across the chunk (N tiles fastest)
   for (int sp = 0; sp < 2; ++sp) {
     const int Ns = ph->Ns[sp];
+    if (traces) {
+      PhExchangeArgs x;
+      memset(&x, 0, sizeof(x));
+      x.nw = w->nw; x.L = ph->L; x.Ns = Ns; x.G = ph->G; x.A = ph->Ahalf[sp].p; x.X = ph->X[sp].p;
+      x.ex = ph->ex.p; x.bg = ph->bgbuf.p; x.accumulate = sp;
+      if ((rc = launch_ph_exchange<T>(x, s))) return rc;
+      continue;
+    }
     for (int w0 = 0; w0 < w->nw; w0 += ph->dchunk) {
       const int nb = std::min(ph->dchunk, w->nw - w0);
+      if (ph->real_half) {
+        RealGemmArgs r;
+        memset(&r, 0, sizeof(r));
+        r.M = ph->G * Ns; r.N = Ns * nb; r.K = ph->L; r.op_t = 1;
+        r.A = ph->Ahalf[sp].p; r.lda = ph->L;
+        r.B = (char*)ph->X[sp].p + ph->esz() * (size_t)w0 * ph->L * Ns; r.ldb = ph->L;
+        r.C = ph->Dbuf.p; r.ldc = (long long)ph->G * Ns;
+        r.alpha = 1.0; r.n_fastest = 1;
+        if ((rc = launch_real_gemm<T>(r, s))) return rc;
+        if ((rc = launch_exchange_trace<T>(nb, ph->G, Ns, ph->Dbuf.p, ph->ex.p + (size_t)w0 * ph->G, sp, s))) return rc;
+        continue;
+      }
       GemmArgs a = gbase();
       a.M = ph->G * Ns; a.N = Ns * nb; a.K = ph->L; a.batch = 1;
       a.A = ph->Ahalf[sp].p; a.lda = ph->L;
@@ -488,15 +543,21 @@ int afqmc_ph_create(afqmc_ctx ctx, const afqmc_ph_desc* d, afqmc_ph* out) {
     }
   }
   const double* hr[2] = {d->half_rot_up, d->half_rot_dn};
+  ph->real_half = 1;
+  for (int sp = 0; sp < 2 && ph->real_half; ++sp)
+    for (long long e = 0, n = (long long)L * ph->Ns[sp] * G; e < n && ph->real_half; ++e)
+      if (hr[sp][2 * e + 1] != 0.0) ph->real_half = 0;
   for (int sp = 0; sp < 2 && !rc; ++sp) {
     const long long n = (long long)L * ph->Ns[sp] * G;
     DevBuf<zd> staging;
     rc = staging.alloc(n);
     if (!rc && hipMemcpy(staging.p, hr[sp], sizeof(zd) * n, hipMemcpyHostToDevice) != hipSuccess) rc = -2;
-    if (!rc) rc = ph->Ahalf[sp].alloc_bytes(es * n);
+    if (!rc) rc = ph->Ahalf[sp].alloc_bytes((ph->real_half ? es / 2 : es) * n);
     if (!rc) {
       unsigned grid = (unsigned)std::min<long long>((n + 255) / 256, 65536);
-      if (ph->fp32) hipLaunchKernelGGL(transpose_half_rot<float>, dim3(grid), dim3(256), 0, 0, L, ph->Ns[sp], G, staging.p, (zf*)ph->Ahalf[sp].p);
+      if (ph->real_half && ph->fp32) hipLaunchKernelGGL(transpose_half_rot_real<float>, dim3(grid), dim3(256), 0, 0, L, ph->Ns[sp], G, (const double*)staging.p, (float*)ph->Ahalf[sp].p);
+      else if (ph->real_half) hipLaunchKernelGGL(transpose_half_rot_real<double>, dim3(grid), dim3(256), 0, 0, L, ph->Ns[sp], G, (const double*)staging.p, (double*)ph->Ahalf[sp].p);
+      else if (ph->fp32) hipLaunchKernelGGL(transpose_half_rot<float>, dim3(grid), dim3(256), 0, 0, L, ph->Ns[sp], G, staging.p, (zf*)ph->Ahalf[sp].p);
       else hipLaunchKernelGGL(transpose_half_rot<double>, dim3(grid), dim3(256), 0, 0, L, ph->Ns[sp], G, staging.p, (zd*)ph->Ahalf[sp].p);
       if (hipDeviceSynchronize() != hipSuccess) rc = -2;
     }
@@ -529,7 +590,7 @@ int afqmc_ph_create(afqmc_ctx ctx, const afqmc_ph_desc* d, afqmc_ph* out) {
   // exchange chunk: keep the (G Ns x Ns) per-walker blocks under 4 GiB
   const long long dper = (long long)G * ph->Nmax * ph->Nmax * (long long)es;
   ph->dchunk = (int)std::max<long long>(1, std::min<long long>(nw, (4ll << 30) / std::max<long long>(dper, 1)));
-  if (!rc) rc = ph->Dbuf.alloc_bytes((size_t)dper * ph->dchunk);
+  if (!rc && !ph_traces(ph)) rc = ph->Dbuf.alloc_bytes((size_t)dper * ph->dchunk);
   if (!rc) rc = ph->qrS.alloc_bytes(sizeof(zd) * (size_t)ph->Nmax * ph->Nmax * nw);
   if (!rc) rc = ph->qrld.alloc(nw);
   if (!rc) rc = ph->qrinfo.alloc(nw);

@@ -210,17 +210,30 @@ __global__ __launch_bounds__(256) void ph_energy_reduce_kernel(int nw, const zd*
   }
 }
 
+// 16 vectors by 16 walker segments a workgroup; the segments are added in order.  With one thread per
+// vector over all walkers 25 waves ran the whole sum: 0.35 ms at 1600 vectors and 1024 walkers, under 0.08 now.
 template <typename T>
-__global__ void ph_g_reduce_kernel(PhEnergyArgs a) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= a.G) return;
+__global__ __launch_bounds__(256) void ph_g_reduce_kernel(PhEnergyArgs a) {
+  __shared__ zd part[2][16][16];
+  const int gl = threadIdx.x & 15, seg = threadIdx.x >> 4, g = blockIdx.x * 16 + gl;
   const cplx<T>* bg = reinterpret_cast<const cplx<T>*>(a.bg);
   zd sb = cmk<double>(0, 0), se = sb;
-  for (int w = 0; w < a.nw; ++w) {
-    if (!a.alive[w]) continue;
-    const zd d = a.den[w];
-    sb = cadd(sb, cmul(to_zd(bg[(long long)w * a.G + g]), d));
-    se = cadd(se, cmul(a.ex[(long long)w * a.G + g], d));
+  if (g < a.G) {
+    const int per = (a.nw + 15) / 16, w1 = min(a.nw, (seg + 1) * per);
+    for (int w = seg * per; w < w1; ++w) {
+      if (!a.alive[w]) continue;
+      const zd d = a.den[w];
+      sb = cadd(sb, cmul(to_zd(bg[(long long)w * a.G + g]), d));
+      se = cadd(se, cmul(a.ex[(long long)w * a.G + g], d));
+    }
+  }
+  part[0][seg][gl] = sb;
+  part[1][seg][gl] = se;
+  __syncthreads();
+  if (seg != 0 || g >= a.G) return;
+  for (int k = 1; k < 16; ++k) {
+    sb = cadd(sb, part[0][k][gl]);
+    se = cadd(se, part[1][k][gl]);
   }
   a.bg_acc[g] = cadd(a.bg_acc[g], sb);
   a.ex_acc[g] = cadd(a.ex_acc[g], se);
@@ -282,8 +295,8 @@ int launch_ph_energy(const PhEnergyArgs& a, hipStream_t s) {
   HIP_LAUNCH_CHECK();
   hipLaunchKernelGGL(ph_energy_reduce_kernel, dim3(1), dim3(256), 0, s, a.nw, a.per_walker, a.sc);
   HIP_LAUNCH_CHECK();
-  if (a.fp32) hipLaunchKernelGGL(ph_g_reduce_kernel<float>, dim3((a.G + 63) / 64), dim3(64), 0, s, a);
-  else hipLaunchKernelGGL(ph_g_reduce_kernel<double>, dim3((a.G + 63) / 64), dim3(64), 0, s, a);
+  if (a.fp32) hipLaunchKernelGGL(ph_g_reduce_kernel<float>, dim3((a.G + 15) / 16), dim3(256), 0, s, a);
+  else hipLaunchKernelGGL(ph_g_reduce_kernel<double>, dim3((a.G + 15) / 16), dim3(256), 0, s, a);
   HIP_LAUNCH_CHECK();
   return 0;
 }

@@ -347,3 +347,38 @@ def test_taylor_fixed_order_zero_freezes_the_first_walkers_order(precision):
         # the dead walker is untouched (held in FP32 on the mixed path)
         dead = wfs[0] if precision == 0 else wfs[0].astype(np.complex64).astype(np.complex128)
         assert np.array_equal(out[0], dead)
+
+
+@pytest.mark.parametrize("L,nup,ndn,G,nw", [(12, 2, 1, 5, 3), (13, 8, 8, 37, 5), (30, 9, 7, 120, 48), (31, 16, 17, 33, 9),
+                                            (45, 24, 25, 64, 3), (64, 32, 33, 70, 2), (50, 40, 41, 21, 3),
+                                            (102, 48, 47, 9, 2), (60, 49, 10, 8, 3), (200, 40, 39, 90, 40)])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_real_half_rotated_vectors_equal_the_general_path(L, nup, ndn, G, nw, precision):
+    """A real trial (real half-rotated vectors: fused traces up to 48 electrons a spin where they fit,
+    else a real product) against the same trial with a phase on each column, which takes the
+    complex products: backgrounds, exchange and energies do not depend on those phases."""
+    rng = np.random.default_rng(L)
+    h = rng.standard_normal((L, L))
+    t = h + h.T
+    v = rng.standard_normal((L, L, G))
+    v = (v + v.transpose(1, 0, 2)) / L
+    model = MoleculeModel(L, nup, ndn, t, t, v, np.zeros(G))
+    orb = np.linalg.qr(rng.standard_normal((L, L)))[0]
+    big = max(nup, ndn)
+    wfs = [orb[:, :big] + 0.1 * crand(rng, L, big) for _ in range(nw)]
+    got = []
+    for phase in (1.0, np.exp(1j * np.arange(1, L + 1))):
+        phi = (orb * phase).astype(complex)
+        prop = PhaselessPropagator(ctx(), model, PhaselessMethod(dt=0.01, walkerSizePerThread=nw),
+                                   phiT=(phi[:, :nup], phi[:, :ndn]), precision=precision, max_walkers=nw)
+        prop.set_onebody(2, np.eye(L), 0j, False)
+        ws = prop.walkers(nw)
+        ws.upload(wfs, np.zeros(nw))
+        prop.reset_measure()
+        prop.measure(ws)
+        e = prop.energy()
+        got.append(np.concatenate([[e["HNum"] / e["den"], e["TNum"] / e["den"]], e["choleskyBgNum"] / e["den"],
+                                   e["choleskyExNum"] / e["den"]]))
+    # D's elements are sums of L products each and the traces sums of up to Ns^2 such elements
+    eps = (1.2e-7 if precision else 2.2e-16) * 8 * np.sqrt(L) * big
+    assert np.max(np.abs(got[0] - got[1])) < eps * np.max(np.abs(got[1])) * 10
