@@ -13,8 +13,10 @@
 //   at a QR after step s: Wt <- Wt R^{-T};  Ybar = B^T Wt_{s+1};  Wt_s = D_s Ybar;
 //   Bbar += Wt_{s+1} (D_s Q_s)^T;  Ubar_i += sum_c Ybar(i,c) Q_s(i,c) D_ii d log D_ii / d U_i.
 // The forward states are checkpointed every ckpt steps and each segment is recomputed (bitwise
-// identically) during the reverse sweep.
+// identically) during the reverse sweep.  Real walkers take the steps between two QRs in one launch
+// (ff_fused.hpp), and keep the states as real numbers.
 #include "cp_internal.hpp"
+#include "ff_fused.hpp"
 
 using namespace cpi;
 
@@ -58,7 +60,7 @@ __global__ void transpose_kernel(long long total, int M, int N, const zd* in, zd
   }
 }
 
-// part[w][i] = sum_c Ybar(i,c) Q(i,c) * D(w,i) * dlogD(w,i)
+// part[w][i] += sum_c Ybar(i,c) Q(i,c) * D(w,i) * dlogD(w,i)
 __global__ void ubar_partial_kernel(int s, unsigned long long key, int nw, int M, int N, double sigma,
                                     const zd* gprime, double dt, const zd* scale, const zd* Yb, const zd* Q, zd* part) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -69,34 +71,44 @@ __global__ void ubar_partial_kernel(int s, unsigned long long key, int nw, int M
   for (int c = 0; c < N; ++c) acc = cadd(acc, cmul(Yb[base + i + (long long)c * M], Q[base + i + (long long)c * M]));
   const double x = field(key, s, nw, M, w, i);
   const zd dl = cmk<double>(sigma * x * gprime[i].re - 0.5 * dt, sigma * x * gprime[i].im);
-  part[(long long)w * M + i] = cmul(cmul(acc, scale[(long long)w * M + i]), dl);
+  zd* o = part + (long long)w * M + i;
+  *o = cadd(*o, cmul(cmul(acc, scale[(long long)w * M + i]), dl));
 }
 
-// out[i] += sum_w part[w][i] (walker order)
-__global__ void sum_walkers_kernel(int nw, int M, const zd* part, zd* out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= M) return;
+// out[e] (+)= sum_w f(w, e): 16 elements by 16 walker segments a workgroup, the segments added in order.
+// One thread an element over all walkers left most of the device idle (117 us for 512 walkers).
+template <typename F>
+__device__ __forceinline__ void sum_over_walkers(int nw, long long per, zd* out, bool accumulate, F f) {
+  __shared__ zd sh[16][16];
+  const int el = threadIdx.x & 15, seg = threadIdx.x >> 4;
+  const long long e = (long long)blockIdx.x * 16 + el;
   zd s = cmk<double>(0, 0);
-  for (int w = 0; w < nw; ++w) s = cadd(s, part[(long long)w * M + i]);
-  out[i] = cadd(out[i], s);
+  if (e < per) {
+    const int chunk = (nw + 15) / 16, w1 = min(nw, (seg + 1) * chunk);
+    for (int w = seg * chunk; w < w1; ++w) s = cadd(s, f(w, e));
+  }
+  sh[seg][el] = s;
+  __syncthreads();
+  if (seg != 0 || e >= per) return;
+  for (int k = 1; k < 16; ++k) s = cadd(s, sh[k][el]);
+  out[e] = accumulate ? cadd(out[e], s) : s;
 }
 
-// out[e] = sum_w c_w * in[w][e] (e < per), walker order
-__global__ void weighted_sum_kernel(int nw, long long per, const zd* c, const zd* in, zd* out) {
-  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= per) return;
-  zd s = cmk<double>(0, 0);
-  for (int w = 0; w < nw; ++w) s = cadd(s, cmul(c[w], in[(long long)w * per + e]));
-  out[e] = s;
+// out[e] = sum_w c_w * in[w][e] (e < per)
+__global__ __launch_bounds__(256) void weighted_sum_kernel(int nw, long long per, const zd* c, const zd* in, zd* out) {
+  sum_over_walkers(nw, per, out, false, [&](int w, long long e) { return cmul(c[w], in[(long long)w * per + e]); });
 }
 
-// out[e] = sum_w in[w][e]
-__global__ void plain_sum_kernel(int nw, long long per, const zd* in, zd* out) {
-  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= per) return;
-  zd s = cmk<double>(0, 0);
-  for (int w = 0; w < nw; ++w) s = cadd(s, in[(long long)w * per + e]);
-  out[e] = s;
+// out[e] (+)= sum_w in[w][e]
+__global__ __launch_bounds__(256) void plain_sum_kernel(int nw, long long per, const zd* in, zd* out, int accumulate) {
+  sum_over_walkers(nw, per, out, accumulate != 0, [&](int w, long long e) { return in[(long long)w * per + e]; });
+}
+
+// u[i] += sum_w c_w mup[w][i] mdn[w][i]
+__global__ __launch_bounds__(256) void udirect_kernel(int nw, int L, const zd* c, const zd* mup, const zd* mdn, zd* u) {
+  sum_over_walkers(nw, L, u, true, [&](int w, long long i) {
+    return cmul(c[w], cmul(mup[(long long)w * L + i], mdn[(long long)w * L + i]));
+  });
 }
 
 // m[w][i] = sum_j theta(i,j) conj(Phi(i,j));  kin[w] (+)= sum_ij theta(i,j) P2(i,j)
@@ -126,28 +138,52 @@ __global__ void kin_kernel(int M, int N, const zd* theta, const zd* p2, zd* kin,
   }
 }
 
-// per walker: E_L, logO; then (one thread, walker order) the weights c_w and E
-__global__ void weights_kernel(int nw, int L, const double* U, const zd* mup, const zd* mdn, const zd* kin,
-                               const zd* logw, const zd* ld0, const zd* ld1, zd* el, zd* logO, zd* c, zd* E) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  double mx = -1e300;
-  for (int w = 0; w < nw; ++w) {
-    zd v = kin[w];
-    for (int i = 0; i < L; ++i) v = cadd(v, cscale(cmul(mup[(long long)w * L + i], mdn[(long long)w * L + i]), U[i]));
-    el[w] = v;
+// per walker: E_L, logO
+__global__ __launch_bounds__(64) void local_energy_kernel(int L, const double* U, const zd* mup, const zd* mdn,
+                                                          const zd* kin, const zd* logw, const zd* ld0, const zd* ld1,
+                                                          zd* el, zd* logO) {
+  const int w = blockIdx.x;
+  zd v = cmk<double>(0, 0);
+  for (int i = threadIdx.x; i < L; i += 64)
+    v = cadd(v, cscale(cmul(mup[(long long)w * L + i], mdn[(long long)w * L + i]), U[i]));
+  v.re = wave_sum(v.re);
+  v.im = wave_sum(v.im);
+  if (threadIdx.x == 0) {
+    el[w] = cadd(kin[w], v);
     logO[w] = cadd(logw[w], cadd(ld0[w], ld1[w]));
-    if (logO[w].re > mx) mx = logO[w].re;
   }
+}
+
+// the weights c_w = O_w / sum O and E, one workgroup, each thread a range of walkers (one thread over
+// all of them took 3.9 ms at 512 walkers on 64 sites)
+__global__ __launch_bounds__(256) void weights_kernel(int nw, const zd* el, const zd* logO, zd* c, zd* E) {
+  __shared__ double shm[256];
+  __shared__ zd sd[256], sn[256];
+  const int tid = threadIdx.x, chunk = (nw + 255) / 256, w0 = min(nw, tid * chunk), w1 = min(nw, w0 + chunk);
+  double mx = -1e300;
+  for (int w = w0; w < w1; ++w)
+    if (logO[w].re > mx) mx = logO[w].re;
+  shm[tid] = mx;
+  __syncthreads();
+  for (int k = 0; k < 256; ++k) mx = shm[k] > mx ? shm[k] : mx;
   zd den = cmk<double>(0, 0), num = den;
-  for (int w = 0; w < nw; ++w) {
+  for (int w = w0; w < w1; ++w) {
     const zd o = cexp_d(cmk<double>(logO[w].re - mx, logO[w].im));
     c[w] = o;
     den = cadd(den, o);
     num = cadd(num, cmul(o, el[w]));
   }
+  sd[tid] = den;
+  sn[tid] = num;
+  __syncthreads();
+  den = num = cmk<double>(0, 0);
+  for (int k = 0; k < 256; ++k) {
+    den = cadd(den, sd[k]);
+    num = cadd(num, sn[k]);
+  }
   const zd inv = cinv(den);
-  for (int w = 0; w < nw; ++w) c[w] = cmul(c[w], inv);
-  *E = cmul(num, inv);
+  for (int w = w0; w < w1; ++w) c[w] = cmul(c[w], inv);
+  if (tid == 0) *E = cmul(num, inv);
 }
 
 // P[w](i,j) = wdkT(i,j) + U_i m_other[w][i] conj(Phi(i,j))
@@ -177,15 +213,6 @@ __global__ void conj_kernel(long long n, const zd* in, zd* out) {
   if (e < n) out[e] = cconj(in[e]);
 }
 
-// u[i] = sum_w c_w mup[w][i] mdn[w][i]
-__global__ void udirect_kernel(int nw, int L, const zd* c, const zd* mup, const zd* mdn, zd* u) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= L) return;
-  zd s = cmk<double>(0, 0);
-  for (int w = 0; w < nw; ++w) s = cadd(s, cmul(c[w], cmul(mup[(long long)w * L + i], mdn[(long long)w * L + i])));
-  u[i] = cadd(u[i], s);
-}
-
 unsigned grid_for(long long n) { return (unsigned)std::min<long long>((n + 255) / 256, 65536); }
 
 // Device scratch of one fixed-field run (spin blocks, FP64).
@@ -201,7 +228,12 @@ struct FF {
   DevBuf<zd> init_logw;
   DevBuf<zd> wt[2], t1[2], t2[2], theta[2], P[2], conjphi[2], oinvT[2], S[2], bb[2];
   DevBuf<zd> m[2], kin, el, logO, c, E, ubar, part, gprime;
+  // real walkers on the fused steps: Q_s of the current segment, slots of Bbar and Ubar
+  bool fused;
+  DevBuf<double> segr[2], bpart[2], upart;
+  bool adjoint;
   int nrq() const { return ckpt / mgs + 1; }
+  int slots() const { return std::min(nw, FF_SLOTS); }
 };
 
 int ff_alloc(FF& f) {
@@ -212,17 +244,24 @@ int ff_alloc(FF& f) {
     const long long n = f.ws[b] * f.nw;
     const long long Nb = cp->Nb[b];
     rc = f.ckw[b].alloc((size_t)(n * f.nseg));
-    if (!rc) rc = f.seg[b].alloc((size_t)(n * nseg_states));
+    if (!rc && f.fused) {
+      if (f.adjoint) {
+        rc = f.segr[b].alloc((size_t)(n * nseg_states));
+        if (!rc) rc = f.bpart[b].alloc((size_t)f.slots() * f.L * f.L);
+      }
+    } else {
+      if (!rc) rc = f.seg[b].alloc((size_t)(n * nseg_states));
+      if (!rc) rc = f.bb[b].alloc((size_t)((long long)f.L * f.L * f.nw));
+      if (!rc) rc = f.t1[b].alloc((size_t)n);
+      if (!rc) rc = f.t2[b].alloc((size_t)n);
+    }
     if (!rc) rc = f.rinv[b].alloc((size_t)(Nb * Nb * f.nw * 2 * f.nrq()));
     if (!rc) rc = f.wt[b].alloc((size_t)n);
-    if (!rc) rc = f.t1[b].alloc((size_t)n);
-    if (!rc) rc = f.t2[b].alloc((size_t)n);
     if (!rc) rc = f.theta[b].alloc((size_t)n);
     if (!rc) rc = f.P[b].alloc((size_t)n);
     if (!rc) rc = f.conjphi[b].alloc((size_t)f.ws[b]);
     if (!rc) rc = f.oinvT[b].alloc((size_t)(Nb * Nb * f.nw));
     if (!rc) rc = f.S[b].alloc((size_t)(Nb * Nb * f.nw));
-    if (!rc) rc = f.bb[b].alloc((size_t)((long long)f.L * f.L * f.nw));
     if (!rc) rc = f.m[b].alloc((size_t)((long long)f.L * f.nw));
   }
   if (!rc) rc = f.ckl.alloc((size_t)f.nw * f.nseg);
@@ -233,7 +272,8 @@ int ff_alloc(FF& f) {
   if (!rc) rc = f.c.alloc(f.nw);
   if (!rc) rc = f.E.alloc(1);
   if (!rc) rc = f.ubar.alloc(f.L);
-  if (!rc) rc = f.part.alloc((size_t)f.nw * f.L);
+  if (!rc && f.fused) rc = f.upart.alloc((size_t)f.slots() * f.L);
+  if (!rc && !f.fused) rc = f.part.alloc((size_t)f.nw * f.L);
   if (!rc) rc = f.gprime.alloc(f.L);
   return rc;
 }
@@ -243,6 +283,27 @@ GemmArgs gb() {
   memset(&a, 0, sizeof(a));
   a.alpha_re = 1.0;
   a.scale_group = 1;
+  return a;
+}
+
+WalkerPanelArgs ff_panel(FF& f, int b, const void* W) {
+  WalkerPanelArgs a;
+  memset(&a, 0, sizeof(a));
+  a.M = f.cp->Mb[b]; a.N = f.cp->Nb[b]; a.nw = f.nw;
+  a.W = W; a.strideW = f.ws[b];
+  return a;
+}
+
+FfFusedArgs ff_fused(FF& f, int b, int s0, int s1, zd* W, double* Q, int q0) {
+  afqmc_cp cp = f.cp;
+  FfFusedArgs a;
+  memset(&a, 0, sizeof(a));
+  a.s0 = s0; a.s1 = s1; a.nw = f.nw; a.M = cp->Mb[b]; a.N = cp->Nb[b]; a.key = f.key;
+  a.sigma = b == 0 ? 1.0 : -1.0; a.dt = cp->dt;
+  a.gamma = cp->gamma.p; a.cdiag = cp->cdiag.p + (b == 0 ? 0 : 3 * f.L);
+  a.B = reinterpret_cast<const double*>(cp->expKr[0][b]);
+  a.W = W; a.Q = Q; a.q0 = q0;
+  a.gprime = f.gprime.p; a.bpart = f.bpart[b].p; a.upart = f.upart.p;
   return a;
 }
 
@@ -263,6 +324,25 @@ int ff_qr(FF& f, int q) {
   for (int pass = 0; pass < 2; ++pass) {
     for (int b = 0; b < 2; ++b) {
       const int Mb = cp->Mb[b], Nb = cp->Nb[b];
+      if (f.fused) {  // in place, R^{-1} straight into its slot
+        zd* ri = q >= 0 ? f.rinv[b].p + ((size_t)q * 2 + pass) * (size_t)Nb * Nb * f.nw
+                        : reinterpret_cast<zd*>(cp->qrS[b].p);
+        WalkerPanelArgs p = ff_panel(f, b, w->wf[b].p);
+        p.out = ri; p.stride_out = (long long)Nb * Nb;
+        if ((rc = launch_walker_gram<double, double>(p, s))) return rc;
+        SmallDenseArgs c;
+        memset(&c, 0, sizeof(c));
+        c.N = Nb; c.batch = f.nw; c.in = ri; c.ld_in = Nb; c.stride_in = (long long)Nb * Nb;
+        c.out = ri; c.ld_out = Nb; c.stride_out = c.stride_in;
+        c.logdet = cp->qrld[b].p; c.info = cp->qrinfo[b].p; c.nsub = Nb; c.alive_div = 1; c.real = 1;
+        if ((rc = launch_chol_inverse<double>(c, s))) return rc;
+        WalkerPanelArgs t = ff_panel(f, b, w->wf[b].p);
+        t.B = ri; t.strideB = (long long)Nb * Nb; t.b_upper = 1;
+        t.out = w->wf[b].p; t.stride_out = t.strideW;
+        if ((rc = launch_walker_times<double, double>(t, s))) return rc;
+        if ((rc = launch_logw_add_real(f.nw, w->logw.p, nullptr, cp->qrld[b].p, nullptr, 0, 1.0, 0.0, s))) return rc;
+        continue;
+      }
       GemmArgs a = gb();
       a.M = Nb; a.N = Nb; a.K = Mb; a.batch = f.nw;
       a.A = w->wf[b].p; a.lda = Mb; a.strideA = f.ws[b];
@@ -300,7 +380,15 @@ int ff_forward(FF& f, int s0, int s1, bool store) {
   afqmc_walkers w = f.w;
   hipStream_t s = cp->ctx->stream;
   int rc;
-  for (int st = s0; st < s1; ++st) {
+  for (int st = s0; f.fused && st < s1;) {  // the steps up to the next QR
+    const int e = std::min(s1, (st / f.mgs + 1) * f.mgs);
+    for (int b = 0; b < 2; ++b)
+      if ((rc = launch_ff_forward(ff_fused(f, b, st, e, (zd*)w->wf[b].p, store ? f.segr[b].p : nullptr, s0), s)))
+        return rc;
+    if (e % f.mgs == 0 && (rc = ff_qr(f, store ? (e - 1 - s0) / f.mgs : -1))) return rc;
+    st = e;
+  }
+  for (int st = s0; !f.fused && st < s1; ++st) {
     if (store)
       for (int b = 0; b < 2; ++b)
         HIP_TRY(hipMemcpyAsync(f.seg[b].p + (size_t)(st - s0) * f.ws[b] * f.nw, w->wf[b].p,
@@ -338,8 +426,10 @@ int ff_terminal(FF& f, bool adjoint) {
                        f.kin.p, b);
     HIP_LAUNCH_CHECK();
   }
-  hipLaunchKernelGGL(weights_kernel, dim3(1), dim3(64), 0, s, f.nw, f.L, cp->U.p, f.m[0].p, f.m[1].p, f.kin.p,
-                     w->logw.p, cp->ldet[0].p, cp->ldet[1].p, f.el.p, f.logO.p, f.c.p, f.E.p);
+  hipLaunchKernelGGL(local_energy_kernel, dim3(f.nw), dim3(64), 0, s, f.L, cp->U.p, f.m[0].p, f.m[1].p, f.kin.p,
+                     w->logw.p, cp->ldet[0].p, cp->ldet[1].p, f.el.p, f.logO.p);
+  HIP_LAUNCH_CHECK();
+  hipLaunchKernelGGL(weights_kernel, dim3(1), dim3(256), 0, s, f.nw, f.el.p, f.logO.p, f.c.p, f.E.p);
   HIP_LAUNCH_CHECK();
   if (!adjoint) return 0;
   for (int b = 0; b < 2; ++b) {
@@ -381,9 +471,35 @@ int ff_terminal(FF& f, bool adjoint) {
     z.C = f.wt[b].p; z.ldc = Mb; z.strideC = f.ws[b];
     if ((rc = launch_cgemm<double>(OP_N, EPI_STORE, z, s))) return rc;
   }
-  hipLaunchKernelGGL(udirect_kernel, dim3((f.L + 63) / 64), dim3(64), 0, s, f.nw, f.L, f.c.p, f.m[0].p, f.m[1].p,
+  hipLaunchKernelGGL(udirect_kernel, dim3((f.L + 15) / 16), dim3(256), 0, s, f.nw, f.L, f.c.p, f.m[0].p, f.m[1].p,
                      f.ubar.p);
   HIP_LAUNCH_CHECK();
+  return 0;
+}
+
+// the reverse steps of segment s0 .. s1-1 on the fused kernels; Wt as below
+int ff_reverse_fused(FF& f, int s0, int s1) {
+  afqmc_cp cp = f.cp;
+  hipStream_t s = cp->ctx->stream;
+  int rc;
+  for (int e = s1; e > s0;) {
+    const int st = std::max(s0, (e - 1) / f.mgs * f.mgs);  // steps st .. e-1 follow the QR at st
+    for (int b = 0; b < 2; ++b) {
+      const int Nb = cp->Nb[b];
+      const long long nn = (long long)Nb * Nb * f.nw;
+      for (int pass = 1; pass >= 0 && e % f.mgs == 0; --pass) {  // Wt <- Wt R2^{-T} R1^{-T}
+        const zd* r = f.rinv[b].p + ((size_t)((e - 1 - s0) / f.mgs) * 2 + pass) * (size_t)nn;
+        hipLaunchKernelGGL(transpose_kernel, dim3(grid_for(nn)), dim3(256), 0, s, nn, Nb, Nb, r, f.oinvT[b].p);
+        HIP_LAUNCH_CHECK();
+        WalkerPanelArgs t = ff_panel(f, b, f.wt[b].p);
+        t.B = f.oinvT[b].p; t.strideB = (long long)Nb * Nb;
+        t.out = f.wt[b].p; t.stride_out = t.strideW;
+        if ((rc = launch_walker_times<double, double>(t, s))) return rc;
+      }
+      if ((rc = launch_ff_reverse(ff_fused(f, b, st, e, f.wt[b].p, f.segr[b].p, s0), s))) return rc;
+    }
+    e = st;
+  }
   return 0;
 }
 
@@ -445,9 +561,6 @@ int ff_reverse_step(FF& f, int st, int s0) {
     hipLaunchKernelGGL(ubar_partial_kernel, dim3((Mb + 63) / 64, f.nw), dim3(64), 0, s, st, f.key, f.nw, Mb, Nb,
                        b == 0 ? 1.0 : -1.0, (const zd*)f.gprime.p, cp->dt, scale, (const zd*)f.t1[b].p, Q, f.part.p);
     HIP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(sum_walkers_kernel, dim3((Mb + 63) / 64), dim3(64), 0, s, f.nw, Mb, (const zd*)f.part.p,
-                       f.ubar.p);
-    HIP_LAUNCH_CHECK();
     // Wt_s = D_s Ybar
     hipLaunchKernelGGL(rowscale_kernel, dim3(grid_for(n)), dim3(256), 0, s, n, Mb, Nb, scale, (const zd*)f.t1[b].p,
                        f.wt[b].p);
@@ -465,11 +578,15 @@ int ff_check(afqmc_cp cp, afqmc_walkers w, int nsteps, int mgs, int ckpt) {
   return 0;
 }
 
-int ff_setup(FF& f, afqmc_cp cp, afqmc_walkers w, int nsteps, int mgs, int ckpt, uint64_t seed) {
+int ff_setup(FF& f, afqmc_cp cp, afqmc_walkers w, int nsteps, int mgs, int ckpt, uint64_t seed, bool adjoint) {
   f.cp = cp; f.w = w; f.nw = w->nw; f.L = cp->L; f.nsteps = nsteps; f.mgs = mgs; f.ckpt = ckpt;
   f.nseg = std::max(1, (nsteps + ckpt - 1) / ckpt);
   f.key = afqmc_seed_mix_host(seed);
   f.ws[0] = w->wsize(0); f.ws[1] = w->wsize(1);
+  f.adjoint = adjoint;
+  // real walkers mean real operators too; wider blocks than the fused kernels take go step by step
+  f.fused = w->real != 0;
+  for (int b = 0; b < 2; ++b) f.fused = f.fused && ff_fused_ok(cp->Mb[b], cp->Nb[b]);
   {
     // the HS factors' U-derivative below assumes constDiag = exp(-dt U_i / 2): mu = h = 0
     std::vector<double> v(f.L);
@@ -494,7 +611,12 @@ int ff_setup(FF& f, afqmc_cp cp, afqmc_walkers w, int nsteps, int mgs, int ckpt,
   HIP_TRY(hipMemcpy(f.gprime.p, gp.data(), sizeof(zd) * f.L, hipMemcpyHostToDevice));
   hipStream_t s = cp->ctx->stream;
   HIP_TRY(hipMemsetAsync(f.ubar.p, 0, sizeof(zd) * f.L, s));
-  for (int b = 0; b < 2; ++b) HIP_TRY(hipMemsetAsync(f.bb[b].p, 0, sizeof(zd) * (size_t)f.L * f.L * f.nw, s));
+  for (int b = 0; b < 2 && adjoint; ++b) {
+    if (f.fused) HIP_TRY(hipMemsetAsync(f.bpart[b].p, 0, sizeof(double) * (size_t)f.slots() * f.L * f.L, s));
+    else HIP_TRY(hipMemsetAsync(f.bb[b].p, 0, sizeof(zd) * (size_t)f.L * f.L * f.nw, s));
+  }
+  if (f.fused) HIP_TRY(hipMemsetAsync(f.upart.p, 0, sizeof(double) * (size_t)f.slots() * f.L, s));
+  else HIP_TRY(hipMemsetAsync(f.part.p, 0, sizeof(zd) * (size_t)f.nw * f.L, s));
   HIP_TRY(hipMemcpyAsync(f.init_logw.p, w->logw.p, sizeof(zd) * f.nw, hipMemcpyDeviceToDevice, s));
   return 0;
 }
@@ -526,7 +648,7 @@ int afqmc_cp_fixed_field_energy(afqmc_cp cp, afqmc_walkers w, int nsteps, int mg
   NOT_CAPTURING();
   ScopedDevice sd(cp->ctx);
   FF f;
-  if ((rc = ff_setup(f, cp, w, nsteps, mgs, mgs, field_seed))) return rc;
+  if ((rc = ff_setup(f, cp, w, nsteps, mgs, mgs, field_seed, false))) return rc;
   if ((rc = ff_ck(f, 0, true))) return rc;
   if ((rc = ff_forward(f, 0, nsteps, false))) return rc;
   if ((rc = ff_terminal(f, false))) return rc;
@@ -548,7 +670,7 @@ int afqmc_cp_fixed_field_adjoint(afqmc_cp cp, afqmc_walkers w, int nsteps, int m
   ScopedDevice sd(cp->ctx);
   hipStream_t s = cp->ctx->stream;
   FF f;
-  if ((rc = ff_setup(f, cp, w, nsteps, mgs, ckpt, field_seed))) return rc;
+  if ((rc = ff_setup(f, cp, w, nsteps, mgs, ckpt, field_seed, true))) return rc;
   // forward with checkpoints at 0, ckpt, 2 ckpt, ...
   for (int k = 0; k < f.nseg; ++k) {
     if ((rc = ff_ck(f, k, true))) return rc;
@@ -562,6 +684,10 @@ int afqmc_cp_fixed_field_adjoint(afqmc_cp cp, afqmc_walkers w, int nsteps, int m
     if (s1 <= s0) continue;
     if ((rc = ff_ck(f, k, false))) return rc;
     if ((rc = ff_forward(f, s0, s1, true))) return rc;
+    if (f.fused) {
+      if ((rc = ff_reverse_fused(f, s0, s1))) return rc;
+      continue;
+    }
     for (int st = s1 - 1; st >= s0; --st)
       if ((rc = ff_reverse_step(f, st, s0))) return rc;
   }
@@ -571,9 +697,13 @@ int afqmc_cp_fixed_field_adjoint(afqmc_cp cp, afqmc_walkers w, int nsteps, int m
   DevBuf<zd> bsum, thsum;
   if ((rc = bsum.alloc((size_t)L * L))) return rc;
   for (int b = 0; b < 2; ++b) {
-    hipLaunchKernelGGL(plain_sum_kernel, dim3(grid_for((long long)L * L)), dim3(256), 0, s, f.nw, (long long)L * L,
-                       (const zd*)f.bb[b].p, bsum.p);
-    HIP_LAUNCH_CHECK();
+    if (f.fused) {
+      if ((rc = launch_ff_sum(f.slots(), L * L, f.bpart[b].p, bsum.p, 0, s))) return rc;
+    } else {
+      hipLaunchKernelGGL(plain_sum_kernel, dim3((L * L + 15) / 16), dim3(256), 0, s, f.nw, (long long)L * L,
+                         (const zd*)f.bb[b].p, bsum.p, 0);
+      HIP_LAUNCH_CHECK();
+    }
     HIP_TRY(hipMemcpyAsync(hb.data(), bsum.p, sizeof(zd) * L * L, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     for (size_t e = 0; e < hb.size(); ++e) {
@@ -586,7 +716,7 @@ int afqmc_cp_fixed_field_adjoint(afqmc_cp cp, afqmc_walkers w, int nsteps, int m
     const int Nb = cp->Nb[b];
     const long long per = (long long)L * Nb;
     if ((rc = thsum.alloc((size_t)per))) return rc;
-    hipLaunchKernelGGL(weighted_sum_kernel, dim3(grid_for(per)), dim3(256), 0, s, f.nw, per, (const zd*)f.c.p,
+    hipLaunchKernelGGL(weighted_sum_kernel, dim3((unsigned)((per + 15) / 16)), dim3(256), 0, s, f.nw, per, (const zd*)f.c.p,
                        (const zd*)f.theta[b].p, thsum.p);
     HIP_LAUNCH_CHECK();
     hth.resize((size_t)per);
@@ -605,6 +735,13 @@ int afqmc_cp_fixed_field_adjoint(afqmc_cp cp, afqmc_walkers w, int nsteps, int m
         mbar[2 * ((size_t)b * L * L + i + (size_t)j * L)] = acc.real();
         mbar[2 * ((size_t)b * L * L + i + (size_t)j * L) + 1] = acc.imag();
       }
+  }
+  if (f.fused) {
+    if ((rc = launch_ff_sum(f.slots(), L, f.upart.p, f.ubar.p, 1, s))) return rc;
+  } else {
+    hipLaunchKernelGGL(plain_sum_kernel, dim3((L + 15) / 16), dim3(256), 0, s, f.nw, (long long)L, (const zd*)f.part.p,
+                       f.ubar.p, 1);
+    HIP_LAUNCH_CHECK();
   }
   std::vector<zd> hu(L);
   zd E;

@@ -99,3 +99,22 @@ def test_torch_autograd_harness():
     _, gt, gU = eng.energy_and_grad(eng.t0, eng.U0)
     assert np.allclose(t.grad.numpy(), gt, rtol=0, atol=0)
     assert float(U.grad) == gU
+
+
+@pytest.mark.parametrize("nx,ny,nup,ndn,nw,nsteps", [(3, 3, 1, 4, 600, 7), (4, 4, 8, 7, 5, 20), (5, 7, 16, 17, 3, 13),
+                                                     (8, 8, 28, 28, 6, 10), (10, 10, 33, 40, 3, 8), (7, 16, 64, 60, 2, 6),
+                                                     (9, 13, 20, 21, 2, 5)])
+def test_fused_real_steps_equal_the_general_path(nx, ny, nup, ndn, nw, nsteps):
+    """A real trial (fused steps up to 112 sites) against the same trial with a phase on each column,
+    which takes the complex path: the energy and its gradient do not depend on those phases.
+    Segments shorter than the run, a last window without a QR, more walkers than slots."""
+    got = []
+    for phase in (0.0, 1.0):
+        eng = FixedFieldHubbard(ctx(), nx, ny, nup, ndn, U=4.0, t2=-0.25, dt=0.02, nw=nw, nsteps=nsteps, mgs=3, ckpt=6)
+        eng.phi = eng.phi * np.exp(1j * phase * np.arange(1, nup + ndn + 1))
+        E, gt, gU = eng.energy_and_grad(eng.t0, eng.U0)
+        assert abs(eng.energy(eng.t0, eng.U0) - E) < 1e-11 * abs(E)
+        got.append(np.concatenate([[E.real, gU], gt]))
+    # sums of L N products of rounding 1.1e-16 each, over nsteps factors, on gradients of the energy's size
+    tol = 1.1e-16 * nx * ny * (nup + ndn) * (nsteps + 10)
+    assert np.max(np.abs(got[0] - got[1])) < tol * max(1.0, np.max(np.abs(got[1])))
