@@ -121,8 +121,8 @@ int step_impl(afqmc_cp cp, afqmc_walkers w, double* force_out, int* aux_out, int
   // so far only workspace has been written: host work on the step's inputs goes here
   if (check && (rc = check())) return rc;
   LogOArgs l = logo_args<T>(cp, w, LOGO_STEP);
-  if ((rc = launch_logo(l, s))) return rc;
-  if ((rc = launch_alive_scan(w->nw, w->alive.p, cp->prefix.p, cp->sc.p, s))) return rc;
+  // given fields draw no uniforms: only the walker-step count advances
+  if ((rc = launch_step_head(l, cp->prefix.p, cp->sc.p, aux_in_dev ? 0 : cp->L, s))) return rc;
   {
     RegionTimer t(cp->ctx, REG_GREEN);
     if ((rc = green_gemm<T>(cp, w, w->wf, w->alive.p, false, w->real))) return rc;
@@ -137,8 +137,6 @@ int step_impl(afqmc_cp cp, afqmc_walkers w, double* force_out, int* aux_out, int
   {
     RegionTimer t(cp->ctx, REG_HS_SAMPLE);
     if ((rc = launch_hs_sample(h, s))) return rc;
-    // given fields draw no uniforms: only the walker-step count advances
-    if ((rc = launch_advance_counter(cp->sc.p, aux_in_dev ? 0 : cp->L, s))) return rc;
   }
   if (cp->diag_only) {
     RegionTimer t(cp->ctx, REG_PROPAGATE);

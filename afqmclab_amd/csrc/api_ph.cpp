@@ -310,8 +310,7 @@ int ph_step_impl(afqmc_ph ph, afqmc_ph_walkers w, double* force_out, double* aux
     if ((rc = ph_overlap<T>(ph, w, w->wf, true, w->alive.p))) return rc;
   }
   LogOArgs l = ph_logo_args(ph, w, LOGO_STEP, w->logw.p);
-  if ((rc = launch_logo(l, s))) return rc;
-  if ((rc = launch_alive_scan(w->nw, w->alive.p, ph->prefix.p, ph->sc.p, s))) return rc;
+  if ((rc = launch_step_head(l, ph->prefix.p, ph->sc.p, 2 * ph->G, s))) return rc;
   {
     RegionTimer t(ph->ctx, REG_PH_FORCE);
     if ((rc = ph_theta<T>(ph, w, w->wf, w->alive.p))) return rc;
@@ -328,7 +327,6 @@ int ph_step_impl(afqmc_ph ph, afqmc_ph_walkers w, double* force_out, double* aux
   {
     RegionTimer t(ph->ctx, REG_PH_SAMPLE);
     if ((rc = launch_ph_sample(a, s))) return rc;
-    if ((rc = launch_advance_counter(ph->sc.p, 2 * ph->G, s))) return rc;
     if ((rc = ph_sample_matrix<T>(ph, w))) return rc;
   }
   {

@@ -39,9 +39,7 @@ struct LogoK {
   static constexpr int NT = 256, WPE = 1;
   __device__ static void run(const BlockIdx3& bk, const LogOArgs& a);
 };
-__device__ __forceinline__ void LogoK::run(const BlockIdx3& bk, const LogOArgs& a) {
-  const int w = bk.x * blockDim.x + threadIdx.x;
-  if (w >= a.nw) return;
+__device__ __forceinline__ void logo_walker(const LogOArgs& a, int w) {
   if (a.mode != LOGO_MEASURE && a.mode != LOGO_ONLY && !a.alive[w]) {
     if (a.mode == LOGO_WEIGHT) a.weight[w] = 0.0;
     return;
@@ -96,43 +94,62 @@ __device__ __forceinline__ void LogoK::run(const BlockIdx3& bk, const LogOArgs& 
   }
 }
 
-// ------------------------------------------------------------------ alive prefix
-struct AliveScanArgs {
-  const int* alive;
+__device__ __forceinline__ void LogoK::run(const BlockIdx3& bk, const LogOArgs& a) {
+  const int w = bk.x * blockDim.x + threadIdx.x;
+  if (w < a.nw) logo_walker(a, w);
+}
+
+// ------------------------------------------------------------------ head of a step
+// The log-overlaps, the alive walkers' prefix, and the step's share of the uniform stream: one
+// workgroup, each thread a contiguous range of walkers.  As three kernels (a log-overlap launch, the
+// scan, and the counter's advance after the sampling) each had a launch and a gap of its own,
+// some 20 us of a small step (10 steps of 128 walkers on 4 x 4 sites with all else alike: 0.08 ms less).
+// Above a walker per thread one CU is too few for the log-overlaps (16.4 us at 2048 walkers), so
+// they keep their own launch there (5.3 us) and logo is 0.
+struct StepHeadArgs {
+  LogOArgs l;
   int* prefix;
   DevScalars* sc;
-  int nw, pad;
+  int per_walker, logo;
 };
-struct AliveScanK {
+struct StepHeadK {
   static constexpr int NT = 1024, WPE = 1;
-  __device__ static void run(const BlockIdx3& bk, const AliveScanArgs& g);
+  __device__ static void run(const BlockIdx3& bk, const StepHeadArgs& g);
 };
-__device__ __forceinline__ void AliveScanK::run(const BlockIdx3& bk, const AliveScanArgs& g) {
-  const int nw = g.nw;
-  const int* alive = g.alive;
-  int* prefix = g.prefix;
-  DevScalars* sc = g.sc;
-
-  __shared__ int part[1024];
-  const int tid = threadIdx.x;
+__device__ __forceinline__ void StepHeadK::run(const BlockIdx3& bk, const StepHeadArgs& g) {
+  __shared__ int part[16];
+  const int nw = g.l.nw, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int* alive = g.l.alive;
   const int chunk = (nw + 1023) / 1024;
-  const int lo = tid * chunk, hi = min(nw, lo + chunk);
+  const int lo = min(nw, tid * chunk), hi = min(nw, lo + chunk);
   int s = 0;
-  for (int i = lo; i < hi; ++i) s += alive[i] ? 1 : 0;
-  part[tid] = s;
+  for (int w = lo; w < hi; ++w) {
+    if (g.logo) logo_walker(g.l, w);
+    s += alive[w] ? 1 : 0;
+  }
+  int p = s;  // inclusive sum over the wave, then over the waves
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(p, o, 64);
+    if (lane >= o) p += v;
+  }
+  if (lane == 63) part[wave] = p;
   __syncthreads();
-  for (int o = 1; o < 1024; o <<= 1) {
-    int v = (tid >= o) ? part[tid - o] : 0;
-    __syncthreads();
-    part[tid] += v;
-    __syncthreads();
+  int base = p - s, total = 0;
+  for (int k = 0; k < 16; ++k) {
+    if (k < wave) base += part[k];
+    total += part[k];
   }
-  int base = part[tid] - s;
-  for (int i = lo; i < hi; ++i) {
-    prefix[i] = base;
-    base += alive[i] ? 1 : 0;
+  for (int w = lo; w < hi; ++w) {
+    g.prefix[w] = base;
+    base += alive[w] ? 1 : 0;
   }
-  if (tid == 1023) sc->alive_count = part[1023];
+  if (tid == 0) {
+    DevScalars* sc = g.sc;
+    sc->alive_count = total;
+    sc->step_base = sc->counter;
+    sc->counter += (unsigned long long)g.per_walker * (unsigned long long)total;
+    sc->walker_steps += (unsigned long long)total;
+  }
 }
 
 // ------------------------------------------------------------------ HS sampling
@@ -223,7 +240,7 @@ __device__ __forceinline__ void HsSampleK<T>::run(const BlockIdx3& bk, const HsS
   if (!a.alive[w]) return;
   __shared__ double sh[16];
   const int L = a.L;
-  const unsigned long long base = a.sc->counter + (unsigned long long)a.prefix[w] * (unsigned long long)L;
+  const unsigned long long base = a.sc->step_base + (unsigned long long)a.prefix[w] * (unsigned long long)L;
   const unsigned long long key = a.sc->key;
   double lp = 0.0;
   zd xg = cmk<double>(0, 0);
@@ -290,22 +307,6 @@ __device__ __forceinline__ void HsSampleK<T>::run(const BlockIdx3& bk, const HsS
     lw.im += sl.im + a.onebody_logw.im;
     a.logw[w] = lw;
   }
-}
-
-struct AdvanceArgs {
-  DevScalars* sc;
-  int per_walker, pad;
-};
-struct AdvanceK {
-  static constexpr int NT = 64, WPE = 1;
-  __device__ static void run(const BlockIdx3& bk, const AdvanceArgs& a);
-};
-__device__ __forceinline__ void AdvanceK::run(const BlockIdx3& bk, const AdvanceArgs& a) {
-  DevScalars* sc = a.sc;
-  const int per_walker = a.per_walker;
-
-  sc->counter += (unsigned long long)per_walker * (unsigned long long)sc->alive_count;
-  sc->walker_steps += (unsigned long long)sc->alive_count;
 }
 
 // ------------------------------------------------------------------ HS 2x2 apply
@@ -1072,23 +1073,22 @@ int launch_logo(const LogOArgs& a, hipStream_t s) {
   return glaunch<LogoK>(a, dim3((a.nw + 255) / 256), dim3(256), 0, s);
 }
 
-int launch_alive_scan(int nw, const int* alive, int* prefix, DevScalars* sc, hipStream_t s) {
-  AliveScanArgs g;
+int launch_step_head(const LogOArgs& a, int* prefix, DevScalars* sc, int per_walker, hipStream_t s) {
+  if (a.nw <= 0) return 0;
+  StepHeadArgs g;
   memset(&g, 0, sizeof(g));
-  g.alive = alive; g.prefix = prefix; g.sc = sc; g.nw = nw;
-  return glaunch<AliveScanK>(g, dim3(1), dim3(1024), 0, s);
+  g.l = a; g.prefix = prefix; g.sc = sc; g.per_walker = per_walker;
+  g.logo = a.nw <= 1024;
+  if (!g.logo) {
+    const int rc = launch_logo(a, s);
+    if (rc) return rc;
+  }
+  return glaunch<StepHeadK>(g, dim3(1), dim3(1024), 0, s);
 }
 
 int launch_hs_sample(const HsSampleArgs& a, hipStream_t s) {
   if (a.fp32) return glaunch<HsSampleK<float>>(a, dim3(a.nw), dim3(256), 0, s);
   return glaunch<HsSampleK<double>>(a, dim3(a.nw), dim3(256), 0, s);
-}
-
-int launch_advance_counter(DevScalars* sc, int per_walker, hipStream_t s) {
-  AdvanceArgs g;
-  memset(&g, 0, sizeof(g));
-  g.sc = sc; g.per_walker = per_walker;
-  return glaunch<AdvanceK>(g, dim3(1), dim3(1), 0, s);
 }
 
 template <typename T>

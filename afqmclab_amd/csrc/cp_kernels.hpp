@@ -10,6 +10,7 @@ struct DevScalars {
   double ET;
   unsigned long long key;      // uniform stream key
   unsigned long long counter;  // next uniform index
+  unsigned long long step_base;  // index of the current step's first uniform
   int alive_count;
   int uniform_overrun;         // set when a kernel asked for a host-provided uniform beyond ulen
   zd den, HNum, KNum, VNum, RNum;
@@ -60,7 +61,9 @@ struct LogOArgs {
 };
 int launch_logo(const LogOArgs& a, hipStream_t s);
 
-int launch_alive_scan(int nw, const int* alive, int* prefix, DevScalars* sc, hipStream_t s);
+// LOGO_STEP of every walker, the alive walkers' prefix and count, and the uniforms of the step:
+// walker w draws per_walker of them from step_base + prefix[w] per_walker on
+int launch_step_head(const LogOArgs& a, int* prefix, DevScalars* sc, int per_walker, hipStream_t s);
 
 struct HsSampleArgs {
   int nw, L, decomp, force_type, nblk, dense;
@@ -82,7 +85,6 @@ struct HsSampleArgs {
   int fp32;
 };
 int launch_hs_sample(const HsSampleArgs& a, hipStream_t s);
-int launch_advance_counter(DevScalars* sc, int per_walker, hipStream_t s);
 
 template <typename T>
 int launch_hs_apply_2x2(int nw, int L, int N, const void* in, void* out, const void* d2x2, hipStream_t s);

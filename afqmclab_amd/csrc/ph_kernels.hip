@@ -32,7 +32,7 @@ __global__ __launch_bounds__(256) void ph_sample_kernel(PhSampleArgs a) {
   typedef cplx<T> ct;
   const ct* bgw = reinterpret_cast<const ct*>(a.bg) + (long long)w * G;
   ct* xsw = reinterpret_cast<ct*>(a.xs) + (long long)w * G;
-  const unsigned long long base = a.sc->counter + (unsigned long long)a.prefix[w] * 2ull * (unsigned long long)G;
+  const unsigned long long base = a.sc->step_base + (unsigned long long)a.prefix[w] * 2ull * (unsigned long long)G;
   const unsigned long long key = a.sc->key;
   zd f2 = cmk<double>(0, 0), xf = f2, xb = f2;
   for (int g = threadIdx.x; g < G; g += blockDim.x) {
