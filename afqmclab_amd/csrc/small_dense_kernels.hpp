@@ -1137,6 +1137,8 @@ __device__ __forceinline__ void GjBK<T, E, NR, NC, WV, NRF, WPEV>::run(const Blo
   }
 }
 
+#include "gj_tiles.hpp"
+
 // Cholesky and R^{-1}, row layout: y[c][r] = element (wave + 16c, lane + 64r).
 template <typename T, typename E, int NR, int NC>
 struct CholK {
@@ -1383,18 +1385,16 @@ template <typename T, typename E>
 int dispatch_registers(int kind, const SmallDenseArgs& a, hipStream_t s) {
   if constexpr (sizeof(E) == 8) {
     if (kind == 0) {
-      // Real matrices: the panel kernel at every size it takes, with as many waves per SIMD as its
-      // registers allow (2048 inversions, FP32 storage: 14 columns 16.7 us against 21.2 for the 2-D
-      // layout, 28: 29.5 against 36.6, 56: 107 with six waves against 151 with four and 163 for the
-      // 1-D layout, 72: 219 with five against 247 with four, 112: 415 with four; the complex panel
-      // kernel takes 1018 us there)
+      // Real matrices: the tiled panel kernel (its comment has both sides' times) from 17 columns on;
+      // up to 16, one update wave, the vector form's shorter chain wins (24 x 256 inversions of 1 to
+      // 16 columns 64 us against 93)
       if (a.N <= 16) return run_gjb<T, E, 1, 4, 1, 1, 8>(a, s);
-      if (a.N <= 32) return run_gjb<T, E, 2, 4, 2, 1, 8>(a, s);
-      if (a.N <= 48) return run_gjb<T, E, 3, 4, 3, 1, 8>(a, s);
-      if (a.N <= 64) return run_gjb<T, E, 4, 4, 4, 1, 6>(a, s);
-      if (a.N <= 80) return run_gjb<T, E, 5, 4, 5, 2, 5>(a, s);
-      if (a.N <= 96) return run_gjb<T, E, 6, 4, 6, 2, 4>(a, s);
-      if (a.N <= 112) return run_gjb<T, E, 7, 4, 7, 2, 4>(a, s);
+      if (a.N <= 32) return run_gjt<T, 2, 8>(a, s);
+      if (a.N <= 48) return run_gjt<T, 3, 8>(a, s);
+      if (a.N <= 64) return run_gjt<T, 4, 8>(a, s);
+      if (a.N <= 80) return run_gjt<T, 5, 6>(a, s);
+      if (a.N <= 96) return run_gjt<T, 6, 6>(a, s);
+      if (a.N <= 112) return run_gjt<T, 7, 6>(a, s);
       if (a.N <= 128) return run_gj<T, E, 2, 8>(a, s);
       return run_gj<T, E, 3, 10, WAVES, 0>(a, s);
     }
