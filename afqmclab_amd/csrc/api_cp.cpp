@@ -755,22 +755,13 @@ int afqmc_cp_walkers_from_trial(afqmc_cp cp, afqmc_walkers w, const double* logw
   REQUIRE(cp && w && w->cp == cp, "invalid argument");
   ScopedDevice sd(cp->ctx);
   hipStream_t s = cp->ctx->stream;
-  HIP_TRY(hipStreamSynchronize(s));
   w->real = cp->real_ops;
-  // phiT into walker 0, then doubling device copies [0, k) -> [k, 2k)
-  for (int b = 0; b < cp->nblk; ++b) {
-    const size_t bytes = cp->esz() * (size_t)w->wsize(b);
-    HIP_TRY(hipMemcpyAsync(w->wf[b].p, cp->phiT[b].p, bytes, hipMemcpyDeviceToDevice, s));
-    for (int k = 1; k < w->nw; k *= 2) {
-      const int m = std::min(k, w->nw - k);
-      HIP_TRY(hipMemcpyAsync(w->wf[b].p + bytes * k, w->wf[b].p, bytes * m, hipMemcpyDeviceToDevice, s));
-    }
-  }
   const zd lw = cmk<double>(logw ? logw[0] : 0.0, logw ? logw[1] : 0.0);
-  std::vector<zd> h(w->nw, lw);
-  std::vector<int> a(w->nw, 1);
-  HIP_TRY(hipMemcpyAsync(w->logw.p, h.data(), sizeof(zd) * w->nw, hipMemcpyHostToDevice, s));
-  HIP_TRY(hipMemcpyAsync(w->alive.p, a.data(), sizeof(int) * w->nw, hipMemcpyHostToDevice, s));
+  for (int b = 0; b < cp->nblk; ++b) {
+    const int rc = launch_broadcast(w->nw, cp->esz() * (size_t)w->wsize(b), cp->phiT[b].p, w->wf[b].p, b == 0 ? w->logw.p : nullptr,
+                                    lw, w->alive.p, s);
+    if (rc) return rc;
+  }
   HIP_TRY(hipStreamSynchronize(s));
   return 0;
 }

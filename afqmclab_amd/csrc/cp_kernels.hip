@@ -1068,6 +1068,40 @@ __global__ void den_sum_kernel(int nw, const zd* den, const int* alive, zd* acc)
 
 }  // namespace
 
+namespace {
+// Each thread keeps one element of the source and stores it for its walkers.  Bound by the stores; as
+// doubling copies a set took 2 + 2 log2(nw) copy commands (18 at 256 walkers, 3 us each, for 24
+// sets 1.5 ms) and two uploads.
+template <typename E>
+__global__ __launch_bounds__(256) void broadcast_kernel(int nw, long long n, const E* __restrict__ src,
+                                                        E* __restrict__ dst, zd* logw, zd lw, int* alive) {
+  const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (logw && blockIdx.x == 0)
+    for (int w = blockIdx.y * 256 + threadIdx.x; w < nw; w += gridDim.y * 256) {
+      logw[w] = lw;
+      alive[w] = 1;
+    }
+  if (e >= n) return;
+  const E v = src[e];
+  for (int w = blockIdx.y; w < nw; w += gridDim.y) dst[(long long)w * n + e] = v;
+}
+}  // namespace
+
+int launch_broadcast(int nw, size_t bytes, const void* src, void* dst, zd* logw, zd lw, int* alive, hipStream_t s) {
+  if (nw <= 0 || (bytes == 0 && !logw)) return 0;
+  const bool wide = bytes % 16 == 0 && ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15) == 0;
+  const long long n = (long long)(bytes / (wide ? 16 : 8));
+  const unsigned gx = (unsigned)std::max<long long>((n + 255) / 256, 1), gy = std::max(1u, std::min((unsigned)nw, 4096u / gx));
+  if (wide)
+    hipLaunchKernelGGL(broadcast_kernel<uint4>, dim3(gx, gy), dim3(256), 0, s, nw, n, (const uint4*)src, (uint4*)dst, logw,
+                       lw, alive);
+  else
+    hipLaunchKernelGGL(broadcast_kernel<uint2>, dim3(gx, gy), dim3(256), 0, s, nw, n, (const uint2*)src, (uint2*)dst, logw,
+                       lw, alive);
+  HIP_LAUNCH_CHECK();
+  return 0;
+}
+
 int launch_logo(const LogOArgs& a, hipStream_t s) {
   if (a.nw <= 0) return 0;
   return glaunch<LogoK>(a, dim3((a.nw + 255) / 256), dim3(256), 0, s);

@@ -60,6 +60,8 @@ struct LogOArgs {
   zd* den;               // MEASURE mode out: exp(logO)
 };
 int launch_logo(const LogOArgs& a, hipStream_t s);
+// dst[w] = src (bytes each, a multiple of 8) for every walker, and with logw: logw[w] = lw, alive[w] = 1
+int launch_broadcast(int nw, size_t bytes, const void* src, void* dst, zd* logw, zd lw, int* alive, hipStream_t s);
 
 // LOGO_STEP of every walker, the alive walkers' prefix and count, and the uniforms of the step:
 // walker w draws per_walker of them from step_base + prefix[w] per_walker on

@@ -179,8 +179,8 @@ def test_graph_of_real_walkers_serves_complex_ones():
 @pytest.mark.parametrize("precision", [0, 1])
 @pytest.mark.parametrize("N", [1, 2, 4, 5, 15, 16, 17, 32, 33, 48, 49, 63, 64, 65, 80, 81, 97, 112, 113, 128, 129, 160])
 def test_gj_real_matches_lapack(precision, N):
-    """Inverse and log-determinant of real matrices in every size class, with a permutation, a singular matrix and a badly scaled one among them.  A backward-stable inverse is
-    within cond * N eps of the exact one; FP32 storage rounds the input-independent result once."""
+    """Inverse and log-determinant of real matrices in every size class, with a permutation, a
+    singular matrix and a badly scaled one among them.  A backward-stable inverse is within cond * N eps of the exact one; FP32 storage rounds the input-independent result once."""
     rng = np.random.default_rng(N)
     A = rng.standard_normal((6, N, N))
     A[1] = np.eye(N)[rng.permutation(N)]
@@ -267,3 +267,29 @@ def test_qr_of_ill_conditioned_real_walkers(precision, nx, ny, nup, ndn):
         assert np.max(np.abs(np.tril(R, -1))) < 20 * eps * size
         assert np.all(np.diag(R).real > 0)
         assert np.max(np.abs(Q @ R - wfs[k])) < 20 * eps * size
+
+
+@pytest.mark.parametrize("nw", [1, 63, 1023, 1024, 1025, 2049])
+def test_step_head_numbers_the_alive_walkers(nw):
+    """The uniforms of a step: walker w draws its own from (alive walkers before it) L on, whatever
+    the population's size and with dead walkers in between; the counter moves by (alive) L."""
+    model = HubbardModel.square(3, 3, 4, 4.0)
+    L = model.L
+    phi = spin_block_trial(model, 2, 2)
+    rng = np.random.default_rng(nw)
+    dead = rng.uniform(size=nw) < 0.3
+    dead[0] = False
+    wfs = [phi + np.where(phi != 0, 0.05 * rng.uniform(-1, 1, phi.shape), 0.0) for _ in range(nw)]
+    got = []
+    for n in (nw, max(1, nw // 2)):  # the first half alone draws the same fields
+        prop = CPPropagator(ctx(), model, CPMethod(dt=0.02, walkerSizePerThread=n), phi, nup=2, spin_blocks=True,
+                            precision=0, max_walkers=n)
+        prop.set_seed(11, 5)
+        ws = prop.walkers(n)
+        ws.upload(wfs[:n], np.zeros(n), (~dead[:n]).astype(np.int32))
+        _, aux = prop.step(ws, record=True)
+        al = ws.alive()
+        assert not np.any(al[dead[:n]])
+        assert prop.counter() == 5 + int(np.sum(al != 0)) * L
+        got.append(np.where(al[:, None] != 0, aux, 0))
+    assert np.array_equal(got[0][:len(got[1])], got[1])
