@@ -1406,12 +1406,15 @@ int dispatch_registers(int kind, const SmallDenseArgs& a, hipStream_t s) {
     // 0.262 ms, four matrices per CU) and 65 to 112 (112: 2.16 against 2.34 ms; 72: 0.309 against
     // 0.343; 96: 1.72 against 1.74), where its registers allow one or two matrices per CU; the 1-D
     // layout otherwise (64: 0.29 against 0.42 for the panel kernel, which fits two matrices per CU
-    // there against the 1-D kernel's four).  The choice depends on N only, so that a grouped call
-    // and the members' own calls do the same arithmetic (the panel kernel's results differ from the
-    // others' in rounding).
+    // there against the 1-D kernel's four).  While all matrices fit the device at two per CU anyway, the
+    // panel kernel's shorter chain wins at 49 to 64 columns too (FP32 storage, 61 columns: 300
+    // matrices 58 us against 95, 512: 62 against 97, 1024: 160 against 154; FP64, 56 columns, 128
+    // matrices: 45 against 55).  The choice depends on the call's own N and batch only, so that a
+    // grouped call and the members' own calls do the same arithmetic (the panel kernel's results
+    // differ from the others' in rounding).
     // a grouped call launches the matrices of all its members together
     const bool many = a.batch > cu_count() || grouping();
-    const bool panels = a.N <= 48 || (a.N > 64 && a.N <= 112);
+    const bool panels = a.N <= 48 || (a.N > 64 && a.N <= 112) || (a.N <= 64 && a.batch <= 2 * cu_count());
     const int layout = a.layout ? a.layout : a.N <= 32 ? 2 : panels ? 3 : 1;
     REQUIRE(layout >= 1 && layout <= 3, "Gauss-Jordan layout %d unknown", layout);
     if (layout == 3 && a.N <= 112) {

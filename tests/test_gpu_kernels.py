@@ -383,3 +383,21 @@ def test_comb_reference_b_exact_weights():
     t, st = comb(ctx(), w, u)
     assert np.array_equal(t, ocomb.popConfiguration(1, w, u))
     assert np.array_equal(np.bincount(t, minlength=100), np.bincount(expect, minlength=100))
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("N", [49, 56, 64])
+@pytest.mark.parametrize("batch", [1, 512, 513])
+def test_gj_at_the_line_between_panels_and_rows(N, batch, precision):
+    """Complex matrices of 49 to 64 columns on both sides of the number that takes the panel kernel:
+    A^{-1} A = 1 to the matrix's conditioning, in every matrix of the batch."""
+    rng = np.random.default_rng(N + batch)
+    A = crand(rng, batch, N, N) + 4 * np.sqrt(N) * np.eye(N)
+    if precision:
+        A = A.astype(np.complex64).astype(np.complex128)
+    inv, ld, info = gj_inverse_masked(A, np.ones(batch, dtype=np.int32), 0, precision)
+    assert not np.any(info)
+    eps = 2.0 ** -53 if precision == 0 else 2.0 ** -24
+    # condition number below 4 by the diagonal shift; N products of rounding eps each
+    assert np.max(np.abs(np.matmul(inv, A) - np.eye(N))) < 8 * N * eps
+    assert np.max(np.abs(ld.real - np.linalg.slogdet(A)[1])) < 1e-11 * N
