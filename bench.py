@@ -49,7 +49,8 @@ def build_workload(nx, ny, nup, ndn, U):
 
 
 def flops_per_walker_step(Ls, nup, ndn, mgs, pop, meas):
-    """Algorithmic flops per walker-step, spin-block form (8 real flops per CMAC)."""
+    """Algorithmic flops per walker-step, spin-block form.  The lattices here have real operators and
+    walkers, so a multiply-add is 2 flops (stored as complex numbers, computed as real ones)."""
     M2N = sum(Ls * Ls * n for n in (nup, ndn))
     MN2 = sum(Ls * n * n for n in (nup, ndn))
     N3 = sum(n ** 3 for n in (nup, ndn))
@@ -58,7 +59,7 @@ def flops_per_walker_step(Ls, nup, ndn, mgs, pop, meas):
     qr = (2 * MN2 - 2.0 / 3.0 * N3) / mgs
     comb = (MN2 + N3 / 3.0) / pop
     measure = (M2N + 2 * MN2 + N3 / 3.0 + 4 * MN) / meas if meas else 0.0
-    return 8.0 * (step + qr + comb + measure), 8.0 * sum(Ls * Ls * n for n in (nup, ndn))
+    return 2.0 * (step + qr + comb + measure), 2.0 * sum(Ls * Ls * n for n in (nup, ndn))
 
 
 def timed_window(thermal, warmup, steps, pop):
@@ -632,7 +633,10 @@ def main():
     fl_ws, fl_prop = flops_per_walker_step(Ls, nup, ndn, sched["mgs"], sched["pop"], sched["meas"])
     # dominant kernel: the one-body propagator GEMM (fused HS scaling), two block launches per step
     tprop, nprop = r["timing"]["propagate"]
-    per_launch_flops = 8.0 * Ls * Ls * nup * args.walkers
+    per_launch_flops = 2.0 * Ls * Ls * nup * args.walkers
+    # walkers read and written once as complex numbers, the HS scale and exp(-dt K)
+    cbytes = 8 if main_path == "mixed" else 16
+    per_launch_bytes = cbytes * args.walkers * (2 * Ls * nup + Ls) + cbytes // 2 * Ls * Ls
     launches = 2 * nprop
     avg_launch_s = tprop / 1e3 / max(launches, 1)
     achieved = per_launch_flops / avg_launch_s / 1e12 if launches else None
@@ -655,22 +659,13 @@ def main():
                    "walkers": args.walkers, "path": main_path, "qr_every": sched["mgs"], "comb_every": sched["pop"],
                    "measure_every": sched["meas"], "thermal_untimed": sched["thermal"],
                    "timed_window": list(r["window"]), "in_window": r["counts"]},
-        "roofline": {"bound": "mfma", "kernel": f"cgemm propagate (exp(-dt K) diag(HS) W), {r['tiles'][0]} tiles",
+        "roofline": {"bound": "mfma", "kernel": "real_gemm propagate (exp(-dt K) diag(HS) W)",
                      "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
                      "frac": (achieved / peak) if achieved else None, "traffic": None,
-                     "avg_launch_ms": avg_launch_s * 1e3, "flops_per_launch": per_launch_flops},
+                     "avg_launch_ms": avg_launch_s * 1e3, "flops_per_launch": per_launch_flops,
+                     "algorithmic_bytes": per_launch_bytes},
         "paths": {},
     }
-    # HBM bytes per launch of the dominant kernel, from the committed rocprofv3 FETCH_SIZE /
-    # WRITE_SIZE passes scaled by the same counters on a plain copy (profiles/)
-    tpath = os.path.join(ROOT, "profiles", "cp_propagate_traffic.json")
-    if os.path.exists(tpath):
-        with open(tpath) as f:
-            tr = json.load(f)
-        by_tile = tr.get("hbm_bytes_per_launch_by_tile", {tr.get("tile"): tr.get("hbm_bytes_per_launch")})
-        if tr.get("workload_walkers") == args.walkers and tr.get("path") == main_path and r["tiles"][0] in by_tile:
-            out["roofline"]["traffic"] = by_tile[r["tiles"][0]]
-            out["roofline"]["algorithmic_bytes"] = tr.get("algorithmic_bytes_per_launch")
     if copy_cal:
         out["copy_calibration"] = copy_cal
     for p, rr in results.items():
