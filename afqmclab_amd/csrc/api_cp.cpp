@@ -221,23 +221,28 @@ int stabilize_impl(afqmc_cp cp, afqmc_walkers w) {
   // 1e-7: their Gram matrix in FP32 (a quarter of the FP64 Gram's time), and the walkers farther
   // than 1e-4 from orthonormal (beyond that Gram's own rounding) take the FP64 check and pass to
   // 1e-8 on their FP64 copy and are rounded again.
-  GroupFork fork;
+  {
+    GroupFork fork;  // each block has a Gram matrix of its own
+    for (int b = 0; b < cp->nblk; ++b) {
+      fork.branch();
+      const int N = cp->Nb[b], M = cp->Mb[b];
+      GemmArgs a;
+      memset(&a, 0, sizeof(a));
+      a.alpha_re = 1.0;
+      a.scale_group = 1;
+      a.M = N; a.N = N; a.K = M; a.batch = w->nw;
+      a.A = w->wf[b].p; a.lda = M; a.strideA = (long long)M * N;
+      a.B = w->wf[b].p; a.ldb = M; a.strideB = (long long)M * N;
+      a.C = cp->qrS[b].p; a.ldc = N; a.strideC = (long long)N * N;
+      a.alive = w->alive.p;
+      a.herm = 1;
+      a.tile = GEMM_TILE_64x64;
+      if ((rc = launch_cgemm<float>(OP_C, EPI_STORE, a, s))) return rc;
+    }
+  }
+  // the blocks share the mask of walkers to redo, the alive flags and the log-weights: one after the other
   for (int b = 0; b < cp->nblk; ++b) {
-    fork.branch();
-    const int N = cp->Nb[b], M = cp->Mb[b];
-    GemmArgs a;
-    memset(&a, 0, sizeof(a));
-    a.alpha_re = 1.0;
-    a.scale_group = 1;
-    a.M = N; a.N = N; a.K = M; a.batch = w->nw;
-    a.A = w->wf[b].p; a.lda = M; a.strideA = (long long)M * N;
-    a.B = w->wf[b].p; a.ldb = M; a.strideB = (long long)M * N;
-    a.C = cp->qrS[b].p; a.ldc = N; a.strideC = (long long)N * N;
-    a.alive = w->alive.p;
-    a.herm = 1;
-    a.tile = GEMM_TILE_64x64;
-    if ((rc = launch_cgemm<float>(OP_C, EPI_STORE, a, s))) return rc;
-    if ((rc = launch_ortho_check_f32(w->nw, N, reinterpret_cast<const zf*>(cp->qrS[b].p), w->alive.p, 1e-4,
+    if ((rc = launch_ortho_check_f32(w->nw, cp->Nb[b], reinterpret_cast<const zf*>(cp->qrS[b].p), w->alive.p, 1e-4,
                                      cp->qr_need.p, s)))
       return rc;
     const CholQrBlock q = qr_block(cp, w, cp->qr64, cp->qr64b, b, 1e-8);

@@ -22,6 +22,15 @@ def ctx():
     return _CTX
 
 
+def gauged(model, step=0.37):
+    """The model with a phase on every site: K_ij exp(i (a_i - a_j)).  Operators, trials and walkers
+    become complex (so the general kernels run); densities, energies and weights stay."""
+    from afqmclab_amd.model import HubbardModel
+    a = step * np.arange(model.L) ** 2 % (2 * np.pi)
+    p = np.exp(1j * np.concatenate([a, a]))
+    return HubbardModel(L=model.L, N=model.N, K=np.asfortranarray(p[:, None] * model.K * p.conj()), U=model.U)
+
+
 def crand(rng, *shape):
     return rng.uniform(-1, 1, shape) + 1j * rng.uniform(-1, 1, shape)
 
