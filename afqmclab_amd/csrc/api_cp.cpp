@@ -963,7 +963,7 @@ int afqmc_cp_onebody(afqmc_cp cp, afqmc_walkers w, int which) {
   if ((rc = launch_logw_const_add(w->nw, w->logw.p, w->alive.p, cp->hop_logw[which], cp->ctx->stream))) return rc;
   HIP_TRY(sync_unless_capturing(cp->ctx->stream));
   capture_note_real(&w->real);
-  capture_note_call([=] { return afqmc_cp_onebody(cp, w, which); });
+  capture_note_call(cp->ctx, [=] { return afqmc_cp_onebody(cp, w, which); });
   return 0;
 }
 
@@ -1008,7 +1008,7 @@ int afqmc_cp_stabilize(afqmc_cp cp, afqmc_walkers w) {
   if (rc) return rc;
   HIP_TRY(sync_unless_capturing(cp->ctx->stream));
   capture_note_real(&w->real);
-  capture_note_call([=] { return afqmc_cp_stabilize(cp, w); });
+  capture_note_call(cp->ctx, [=] { return afqmc_cp_stabilize(cp, w); });
   return 0;
 }
 
@@ -1063,7 +1063,7 @@ int afqmc_cp_step(afqmc_cp cp, afqmc_walkers w, double* force_out, int* aux_out)
   int rc = DISPATCH(cp, step_impl, cp, w, force_out, aux_out);
   if (rc) return rc;
   capture_note_real(&w->real);
-  capture_note_call([=] { return afqmc_cp_step(cp, w, nullptr, nullptr); });
+  capture_note_call(cp->ctx, [=] { return afqmc_cp_step(cp, w, nullptr, nullptr); });
   return 0;
 }
 
@@ -1074,7 +1074,7 @@ int afqmc_cp_pop_control(afqmc_cp cp, afqmc_walkers w, double* weights_out, int*
   int rc = DISPATCH(cp, pop_control_impl, cp, w, weights_out, table_out, stats);
   if (rc) return rc;
   capture_note_real(&w->real);
-  capture_note_call([=] { return afqmc_cp_pop_control(cp, w, nullptr, nullptr, nullptr); });
+  capture_note_call(cp->ctx, [=] { return afqmc_cp_pop_control(cp, w, nullptr, nullptr, nullptr); });
   return 0;
 }
 
@@ -1137,7 +1137,7 @@ int afqmc_cp_measure(afqmc_cp cp, afqmc_walkers w) {
   int rc = DISPATCH(cp, measure_impl, cp, w);
   if (rc) return rc;
   capture_note_real(&w->real);
-  capture_note_call([=] { return afqmc_cp_measure(cp, w); });
+  capture_note_call(cp->ctx, [=] { return afqmc_cp_measure(cp, w); });
   return 0;
 }
 
@@ -1167,7 +1167,7 @@ int afqmc_cp_reset_measure(afqmc_cp cp) {
   ScopedDevice sd(cp->ctx);
   int rc = launch_reset_measure(cp->sc.p, cp->site_acc.p, cp->L, cp->ctx->stream);
   if (rc) return rc;
-  capture_note_call([=] { return afqmc_cp_reset_measure(cp); });
+  capture_note_call(cp->ctx, [=] { return afqmc_cp_reset_measure(cp); });
   return 0;
 }
 
@@ -1177,7 +1177,7 @@ int afqmc_cp_adjust_ET(afqmc_cp cp) {
   int rc = launch_set_et_from_energy(cp->sc.p, cp->ctx->stream);
   if (!rc) rc = launch_reset_measure(cp->sc.p, cp->site_acc.p, cp->L, cp->ctx->stream);
   if (rc) return rc;
-  capture_note_call([=] { return afqmc_cp_adjust_ET(cp); });
+  capture_note_call(cp->ctx, [=] { return afqmc_cp_adjust_ET(cp); });
   return 0;
 }
 
@@ -1296,14 +1296,14 @@ int afqmc_cp_group_step(afqmc_cp_group g) {
   int rc = run_grouped(g, [&](afqmc_cp cp, afqmc_walkers w) {
     return g->fp32 ? step_impl<float>(cp, w, nullptr, nullptr) : step_impl<double>(cp, w, nullptr, nullptr);
   });
-  if (!rc) capture_note_call([=] { return afqmc_cp_group_step(g); });
+  if (!rc) capture_note_call(g->ctx, [=] { return afqmc_cp_group_step(g); });
   return rc;
 }
 
 int afqmc_cp_group_stabilize(afqmc_cp_group g) {
   REQUIRE(g, "null argument");
   int rc = run_grouped(g, [&](afqmc_cp cp, afqmc_walkers w) { return stabilize_impl(cp, w); });
-  if (!rc) capture_note_call([=] { return afqmc_cp_group_stabilize(g); });
+  if (!rc) capture_note_call(g->ctx, [=] { return afqmc_cp_group_stabilize(g); });
   return rc;
 }
 
@@ -1313,7 +1313,7 @@ int afqmc_cp_group_pop_control(afqmc_cp_group g) {
     return g->fp32 ? pop_control_impl<float>(cp, w, nullptr, nullptr, nullptr)
                    : pop_control_impl<double>(cp, w, nullptr, nullptr, nullptr);
   });
-  if (!rc) capture_note_call([=] { return afqmc_cp_group_pop_control(g); });
+  if (!rc) capture_note_call(g->ctx, [=] { return afqmc_cp_group_pop_control(g); });
   return rc;
 }
 

@@ -49,6 +49,12 @@ __global__ void transpose_half_rot_real(int L, int Ns, int G, const double* in, 
     out[e] = (T)in[2 * (j + (long long)i * Ns + g * (long long)Ns * L)];
   }
 }
+// a and b = 0 (a kernel where a caller may capture: memset nodes of a graph have given wrong results on
+// later replays)
+__global__ void clear_kernel(int n, zd* a, zd* b) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) a[i] = b[i] = cmk<double>(0, 0);
+}
 }  // namespace
 
 struct afqmc_ph_s {
@@ -967,14 +973,21 @@ int afqmc_ph_step(afqmc_ph ph, afqmc_ph_walkers w, double* force_out, double* au
 
 int afqmc_ph_pop_control(afqmc_ph ph, afqmc_ph_walkers w, double* weights_out, int* table_out, double* stats) {
   REQUIRE(ph && w && w->ph == ph, "invalid argument");
+  REQUIRE(!capturing() || (!weights_out && !table_out && !stats), "a captured comb cannot return outputs");
   ScopedDevice sdv(ph->ctx);
-  return PH_DISPATCH(ph, ph_pop_control_impl, ph, w, weights_out, table_out, stats);
+  int rc = PH_DISPATCH(ph, ph_pop_control_impl, ph, w, weights_out, table_out, stats);
+  if (rc) return rc;
+  capture_note_call(ph->ctx, [=] { return afqmc_ph_pop_control(ph, w, nullptr, nullptr, nullptr); });
+  return 0;
 }
 
 int afqmc_ph_measure(afqmc_ph ph, afqmc_ph_walkers w) {
   REQUIRE(ph && w && w->ph == ph, "invalid argument");
   ScopedDevice sdv(ph->ctx);
-  return PH_DISPATCH(ph, ph_measure_impl, ph, w);
+  int rc = PH_DISPATCH(ph, ph_measure_impl, ph, w);
+  if (rc) return rc;
+  capture_note_call(ph->ctx, [=] { return afqmc_ph_measure(ph, w); });
+  return 0;
 }
 
 int afqmc_ph_energy(afqmc_ph ph, double* out, double* bg_num, double* ex_num) {
@@ -990,14 +1003,21 @@ int afqmc_ph_energy(afqmc_ph ph, double* out, double* bg_num, double* ex_num) {
   return 0;
 }
 
-int afqmc_ph_reset_measure(afqmc_ph ph) {
-  REQUIRE(ph, "null argument");
-  ScopedDevice sdv(ph->ctx);
+static int reset_measure(afqmc_ph ph) {
   hipStream_t s = ph->ctx->stream;
   int rc = launch_reset_measure(ph->sc.p, ph->bg_acc.p, 0, s);
   if (rc) return rc;
-  HIP_TRY(hipMemsetAsync(ph->bg_acc.p, 0, sizeof(zd) * ph->G, s));
-  HIP_TRY(hipMemsetAsync(ph->ex_acc.p, 0, sizeof(zd) * ph->G, s));
+  hipLaunchKernelGGL(clear_kernel, dim3((ph->G + 255) / 256), dim3(256), 0, s, ph->G, ph->bg_acc.p, ph->ex_acc.p);
+  HIP_LAUNCH_CHECK();
+  return 0;
+}
+
+int afqmc_ph_reset_measure(afqmc_ph ph) {
+  REQUIRE(ph, "null argument");
+  ScopedDevice sdv(ph->ctx);
+  int rc = reset_measure(ph);
+  if (rc) return rc;
+  capture_note_call(ph->ctx, [=] { return afqmc_ph_reset_measure(ph); });
   return 0;
 }
 
@@ -1005,8 +1025,10 @@ int afqmc_ph_adjust_ET(afqmc_ph ph) {
   REQUIRE(ph, "null argument");
   ScopedDevice sdv(ph->ctx);
   int rc = launch_set_et_from_energy(ph->sc.p, ph->ctx->stream);
+  if (!rc) rc = reset_measure(ph);
   if (rc) return rc;
-  return afqmc_ph_reset_measure(ph);
+  capture_note_call(ph->ctx, [=] { return afqmc_ph_adjust_ET(ph); });
+  return 0;
 }
 
 }  // extern "C"

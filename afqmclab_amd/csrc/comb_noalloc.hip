@@ -80,5 +80,6 @@ extern "C" int afqmc_comb_noalloc(afqmc_ctx ctx, int nw, const double* weight, c
     hipLaunchKernelGGL(noalloc_stats_kernel, dim3(1), dim3(64), 0, s, sc, stats);
     HIP_LAUNCH_CHECK();
   }
+  capture_note_call(ctx, [=] { return afqmc_comb_noalloc(ctx, nw, weight, uniforms, table, stats); });
   return 0;
 }

@@ -47,13 +47,21 @@ extern thread_local CaptureSession* g_capture;
 inline bool capturing() { return g_capture != nullptr; }
 inline hipError_t sync_unless_capturing(hipStream_t s) { return g_capture ? hipSuccess : hipStreamSynchronize(s); }
 void capture_note_pair(DevBuf<char>* a, DevBuf<char>* b);
+// whether work on this context goes into the open capture (its origin or a member)
+inline bool captured_on(afqmc_ctx c) {
+  if (!g_capture || c == g_capture->origin) return g_capture != nullptr;
+  for (afqmc_ctx m : g_capture->members)
+    if (m == c) return true;
+  return false;
+}
 // notes the `real` flag a captured call relies on
 inline void capture_note_real(const int* real) {
   if (g_capture) g_capture->real_flags.push_back({real, *real});
 }
-// records a call that has just been captured
-inline void capture_note_call(std::function<int()> call) {
-  if (g_capture) g_capture->calls.push_back(std::move(call));
+// Records a call on context c that has just been captured.  Every entry point whose work a capture
+// records does so, walkers or not: a graph whose calls are made again makes all of them.
+inline void capture_note_call(afqmc_ctx c, std::function<int()> call) {
+  if (captured_on(c)) g_capture->calls.push_back(std::move(call));
 }
 #define NOT_CAPTURING() REQUIRE(!capturing(), "%s cannot be recorded into a graph (it synchronises)", __func__)
 

@@ -46,11 +46,16 @@ int afqmc_ctx_get_timing(afqmc_ctx ctx, double* total_ms, long long* count, int 
 /* HIP-graph capture of enqueue-only calls (no reference counterpart: the reference launches
  * nothing).  Between begin and end, the calls made on this thread are recorded instead of run:
  * afqmc_cp_step (without records), afqmc_cp_stabilize, afqmc_cp_pop_control (without outputs),
- * afqmc_cp_measure, afqmc_cp_onebody, afqmc_cp_reset_measure, afqmc_cp_adjust_ET.  Calls that
- * return data to the host fail while a capture is open.  begin_group also records work issued on
+ * afqmc_cp_measure, afqmc_cp_onebody, afqmc_cp_reset_measure, afqmc_cp_adjust_ET, the calls of a group
+ * of runs, afqmc_comb_noalloc, and of the phaseless calls afqmc_ph_measure (with a dense one-body
+ * operator), afqmc_ph_pop_control (without outputs), afqmc_ph_reset_measure and afqmc_ph_adjust_ET.
+ * Calls that return data to the host fail while a capture is open.  begin_group also records work issued on
  * the member contexts (one stream each; e.g. independent lattices), which become parallel
  * branches of one graph.  afqmc_graph_launch enqueues the whole graph on the origin's stream
- * (asynchronous).  Walker sets and propagators used in a graph must outlive it. */
+ * (asynchronous).  Where a walker set whose elements were all real at the capture has since become
+ * complex (uploaded, hs_apply), the kernels recorded for it do not hold: a launch then makes all the recorded
+ * calls again, in their order, with the same results.  Walker sets, propagators, groups and device
+ * arrays used in a graph must outlive it. */
 int afqmc_capture_begin(afqmc_ctx ctx);
 int afqmc_capture_begin_group(afqmc_ctx origin, int n, const afqmc_ctx* members);
 int afqmc_capture_end(afqmc_ctx origin, afqmc_graph* out);

@@ -7,9 +7,11 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
+from afqmclab_amd._lib import check, lib  # noqa: E402
 from afqmclab_amd.cp import Context, CPGroup, CPMethod, CPPropagator  # noqa: E402
 from afqmclab_amd.model import HubbardModel, free_electron_trial, spin_block_trial  # noqa: E402
 from tests.gpu_util import ctx, gauged  # noqa: E402
+from tests.test_zz_no_alloc import DevArray, comb_host  # noqa: E402
 
 
 # the Green GEMM's epilogue needs the 64-column tiles
@@ -190,3 +192,125 @@ def test_grouped_qr_of_ill_conditioned_walkers_equals_own_calls(precision, phase
             q = a[0][k]
             assert np.max(np.abs(q.conj().T @ q - np.eye(2 * nup))) < (1e-12 if precision == 0 else 1.1e-4), k
     grp.close()
+
+
+class Comb:
+    """afqmc_comb_noalloc on device arrays: call() enqueues it, check() compares with afqmc_comb."""
+
+    def __init__(self, c, nw, seed):
+        rng = np.random.default_rng(seed)
+        self.c, self.w, self.u = c, rng.uniform(0, 5, nw), rng.uniform(0, 1, nw)
+        self.dev = [DevArray(a) for a in (self.w, self.u, np.full(nw, -7, dtype=np.int32), np.zeros(3))]
+        self.ref = comb_host(self.w, self.u)
+
+    def call(self):
+        dw, du, dt, ds = self.dev
+        check(lib().afqmc_comb_noalloc(self.c.h, len(self.w), dw.p, du.p, dt.p, ds.p))
+
+    def check(self):
+        """The results so far, which are then wiped."""
+        dt, ds = self.dev[2:]
+        assert np.array_equal(dt.get(), self.ref[0]) and np.array_equal(ds.get(), self.ref[1])
+        for d in (dt, ds):
+            d.put(np.full_like(d.host, -7))
+
+
+@pytest.mark.parametrize("form", ["context", "members", "group"])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_graph_of_real_walkers_makes_all_its_calls_for_complex_ones(form, precision):
+    """A graph captured while its sets are real, launched after one of them became complex: every
+    recorded call is made again, those on other sets and those without walkers (the comb on device
+    buffers) included, from one context, from member contexts and for a group's calls.  Identical to
+    eager calls, real and complex walkers in turn (one restabilisation a block, so the walkers' buffers
+    change parity between the launches)."""
+    shapes = [(4, 4, 5, 4.0), (6, 4, 9, 3.0)]
+    origin = Context(0)
+    gctx = [Context(0) for _ in shapes] if form == "members" else [origin] * len(shapes)
+    gsets = [make(c, *s, precision=precision, seed=21 + i) for i, (c, s) in enumerate(zip(gctx, shapes))]
+    esets = [make(ctx(), *s, precision=precision, seed=21 + i) for i, s in enumerate(shapes)]
+    grp = CPGroup(gsets) if form == "group" else None
+    comb = Comb(gctx[1], 500, 8)
+    start = [w.download()[0] for _, w in gsets]
+
+    def block(sets, grp=None):
+        if grp is None:
+            for p, w in sets:
+                block_of_work(p, w)
+            return
+        for _ in range(3):
+            grp.step()
+        grp.stabilize()
+        grp.pop_control()
+        for p, w in sets:
+            p.measure(w)
+
+    origin.capture_begin(members=gctx if form == "members" else ())
+    block(gsets, grp)
+    comb.call()
+    g = origin.capture_end()
+    for theta in (0.0, 0.6, 0.0, 0.0, 0.6, 0.6):
+        up = [w.copy() for w in start]
+        up[0][:, :, 0] *= np.exp(1j * theta)  # the second set stays real
+        for sets in (gsets, esets):
+            for (p, w), x in zip(sets, up):
+                w.upload(x, np.full(w.nw, -1j * theta if x is up[0] else 0.0))
+                p.reset_measure()
+        for _ in range(2):
+            g.launch()
+            block(esets)
+            for c in [origin] + gctx:
+                c.synchronize()
+            comb.check()
+            for (p1, w1), (p2, w2) in zip(gsets, esets):
+                same(state(p1, w1), state(p2, w2))
+    g.close()
+    if grp:
+        grp.close()
+
+
+def test_graph_with_phaseless_calls_makes_them_for_complex_walkers_too():
+    """The phaseless measurement, comb and resets recorded beside a real constraint-path set: made by
+    the graph and, after that set became complex, by the repeated calls, as eagerly."""
+    from tests.test_gpu_ph import make_case
+    c = Context(0)
+    cp, cw = make(c, 4, 4, 5, 4.0)
+    got = []
+    for _ in range(2):  # on the shared context
+        _, dm, _, prop, ws, *_ = make_case(seed=4)
+        B, lw = dm.exp_minus_alpha_k(-0.025)
+        prop.set_onebody(2, B, lw, False)
+        got.append((prop, ws))
+    shared = ctx()
+    real = cw.download()[0]
+
+    def work(prop, ws, k):
+        if k:
+            prop.adjust_ET()
+        else:
+            prop.reset_measure()
+        prop.measure(ws)
+        prop.pop_control(ws)
+        prop.measure(ws)
+
+    graphs = []
+    for k in range(2):
+        c.capture_begin(members=[shared])
+        cp.step(cw)
+        work(*got[0], k)
+        graphs.append(c.capture_end())
+    for theta in (0.0, 0.6, 0.0):
+        up = real.copy()
+        up[:, :, 0] *= np.exp(1j * theta)
+        cw.upload(up, np.full(cw.nw, -1j * theta))
+        for k in (0, 1, 1):
+            graphs[k].launch()
+            work(*got[1], k)
+            c.synchronize()
+            shared.synchronize()
+            (p1, w1), (p2, w2) = got
+            same(w1.download(), w2.download())
+            e1, e2 = p1.energy(), p2.energy()
+            assert all(np.array_equal(e1[n], e2[n]) for n in e1)
+            assert p1.get_ET() == p2.get_ET() and p1.counter() == p2.counter()
+    for g in graphs:
+        g.close()

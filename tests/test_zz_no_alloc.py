@@ -27,6 +27,9 @@ class DevArray:
         assert _hip.hipMalloc(C.byref(self.p), max(self.host.nbytes, 16)) == 0
         assert _hip.hipMemcpy(self.p, self.host.ctypes.data, self.host.nbytes, H2D) == 0
 
+    def put(self, host):
+        assert _hip.hipMemcpy(self.p, np.ascontiguousarray(host).ctypes.data, self.host.nbytes, H2D) == 0
+
     def get(self):
         out = np.empty_like(self.host)
         assert _hip.hipMemcpy(out.ctypes.data, self.p, out.nbytes, D2H) == 0
