@@ -961,7 +961,7 @@ int afqmc_cp_onebody(afqmc_cp cp, afqmc_walkers w, int which) {
       return rc;
   }
   if ((rc = launch_logw_const_add(w->nw, w->logw.p, w->alive.p, cp->hop_logw[which], cp->ctx->stream))) return rc;
-  HIP_TRY(sync_unless_capturing(cp->ctx->stream));
+  HIP_TRY(sync_unless_enqueuing(cp->ctx->stream));
   capture_note_real(&w->real);
   capture_note_call(cp->ctx, [=] { return afqmc_cp_onebody(cp, w, which); });
   return 0;
@@ -1006,7 +1006,7 @@ int afqmc_cp_stabilize(afqmc_cp cp, afqmc_walkers w) {
   ScopedDevice sd(cp->ctx);
   int rc = stabilize_impl(cp, w);
   if (rc) return rc;
-  HIP_TRY(sync_unless_capturing(cp->ctx->stream));
+  HIP_TRY(sync_unless_enqueuing(cp->ctx->stream));
   capture_note_real(&w->real);
   capture_note_call(cp->ctx, [=] { return afqmc_cp_stabilize(cp, w); });
   return 0;

@@ -263,6 +263,7 @@ int launch_reset_measure(DevScalars* sc, zd* site_acc, int L, hipStream_t s) {
 }
 
 thread_local CaptureSession* g_capture = nullptr;
+thread_local bool g_reissuing = false;
 
 void capture_note_pair(DevBuf<char>* a, DevBuf<char>* b) {
   if (!g_capture) return;
@@ -476,8 +477,10 @@ int afqmc_graph_launch(afqmc_graph g) {
       for (afqmc_ctx m : g->members) HIP_TRY(hipStreamWaitEvent(m->stream, g->ev, 0));
     }
     int rc = 0;
+    g_reissuing = true;
     for (auto& call : g->calls)
       if (!rc) rc = call();
+    g_reissuing = false;
     for (afqmc_ctx m : g->members) {
       HIP_TRY(hipEventRecord(g->ev, m->stream));
       HIP_TRY(hipStreamWaitEvent(s, g->ev, 0));

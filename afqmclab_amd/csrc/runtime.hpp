@@ -45,7 +45,11 @@ struct CaptureSession {
 };
 extern thread_local CaptureSession* g_capture;
 inline bool capturing() { return g_capture != nullptr; }
-inline hipError_t sync_unless_capturing(hipStream_t s) { return g_capture ? hipSuccess : hipStreamSynchronize(s); }
+// set while afqmc_graph_launch makes a graph's calls again: it enqueues only, as the graph would
+extern thread_local bool g_reissuing;
+inline hipError_t sync_unless_enqueuing(hipStream_t s) {
+  return g_capture || g_reissuing ? hipSuccess : hipStreamSynchronize(s);
+}
 void capture_note_pair(DevBuf<char>* a, DevBuf<char>* b);
 // whether work on this context goes into the open capture (its origin or a member)
 inline bool captured_on(afqmc_ctx c) {

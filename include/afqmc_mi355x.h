@@ -54,7 +54,7 @@ int afqmc_ctx_get_timing(afqmc_ctx ctx, double* total_ms, long long* count, int 
  * branches of one graph.  afqmc_graph_launch enqueues the whole graph on the origin's stream
  * (asynchronous).  Where a walker set whose elements were all real at the capture has since become
  * complex (uploaded, hs_apply), the kernels recorded for it do not hold: a launch then makes all the recorded
- * calls again, in their order, with the same results.  Walker sets, propagators, groups and device
+ * calls again, in their order, with the same results (enqueued only, too).  Walker sets, propagators, groups and device
  * arrays used in a graph must outlive it. */
 int afqmc_capture_begin(afqmc_ctx ctx);
 int afqmc_capture_begin_group(afqmc_ctx origin, int n, const afqmc_ctx* members);
