@@ -209,7 +209,6 @@ int ph_taylor_pass(afqmc_ph ph, afqmc_ph_walkers w, DevBuf<char>& wf, const void
   const long long n = w->wsize();
   const size_t bytes = ph->esz() * n * w->nw;
   int rc;
-  REQUIRE(!capturing(), "the Taylor series of exp(A) W cannot be captured (its length depends on the walkers)");
   // tmp <- W (the accumulated sum); the first product reads W itself
   HIP_TRY(hipMemcpyAsync(w->tmp.p, wf.p, bytes, hipMemcpyDeviceToDevice, s));
   HIP_TRY(hipMemcpyAsync(ph->active.p, mask, sizeof(int) * w->nw, hipMemcpyDeviceToDevice, s));
@@ -660,6 +659,7 @@ int afqmc_ph_destroy(afqmc_ph ph) {
 
 int afqmc_ph_set_onebody(afqmc_ph ph, int which, const double* matrix, const double* logw, int is_log) {
   REQUIRE(ph && matrix && logw, "null argument");
+  NOT_CAPTURED(ph->ctx);
   REQUIRE(which >= 0 && which <= 2, "which must be 0, 1 or 2");
   ScopedDevice sdv(ph->ctx);
   HIP_TRY(hipStreamSynchronize(ph->ctx->stream));
@@ -674,6 +674,7 @@ int afqmc_ph_set_onebody(afqmc_ph ph, int which, const double* matrix, const dou
 
 int afqmc_ph_set_background(afqmc_ph ph, const double* bg) {
   REQUIRE(ph && bg, "null argument");
+  NOT_CAPTURED(ph->ctx);
   ScopedDevice sdv(ph->ctx);
   HIP_TRY(hipStreamSynchronize(ph->ctx->stream));
   std::copy(bg, bg + ph->G, ph->h_bg.begin());
@@ -719,6 +720,7 @@ int afqmc_ph_walkers_destroy(afqmc_ph_walkers w) {
 
 int afqmc_ph_walkers_upload(afqmc_ph_walkers w, const double* wf, const double* logw, const int* alive) {
   REQUIRE(w && wf && logw, "null argument");
+  NOT_CAPTURED(w->ph->ctx);
   afqmc_ph ph = w->ph;
   ScopedDevice sdv(ph->ctx);
   HIP_TRY(hipStreamSynchronize(ph->ctx->stream));
@@ -739,6 +741,7 @@ int afqmc_ph_walkers_upload(afqmc_ph_walkers w, const double* wf, const double* 
 
 int afqmc_ph_walkers_download(afqmc_ph_walkers w, double* wf, double* logw, int* alive) {
   REQUIRE(w, "null argument");
+  NOT_CAPTURED(w->ph->ctx);
   afqmc_ph ph = w->ph;
   ScopedDevice sdv(ph->ctx);
   HIP_TRY(hipStreamSynchronize(ph->ctx->stream));
@@ -766,6 +769,7 @@ static int ph_scalars(afqmc_ph ph, DevScalars* h, bool write) {
 
 int afqmc_ph_set_seed(afqmc_ph ph, uint64_t seed, uint64_t counter) {
   REQUIRE(ph, "null argument");
+  NOT_CAPTURED(ph->ctx);
   ScopedDevice sdv(ph->ctx);
   DevScalars h;
   int rc = ph_scalars(ph, &h, false);
@@ -777,6 +781,7 @@ int afqmc_ph_set_seed(afqmc_ph ph, uint64_t seed, uint64_t counter) {
 
 int afqmc_ph_get_counter(afqmc_ph ph, uint64_t* counter, uint64_t* walker_steps) {
   REQUIRE(ph && counter, "null argument");
+  NOT_CAPTURED(ph->ctx);
   ScopedDevice sdv(ph->ctx);
   DevScalars h;
   int rc = ph_scalars(ph, &h, false);
@@ -789,6 +794,7 @@ int afqmc_ph_get_counter(afqmc_ph ph, uint64_t* counter, uint64_t* walker_steps)
 
 int afqmc_ph_get_qr_stats(afqmc_ph ph, uint64_t* shifted, uint64_t* killed) {
   REQUIRE(ph && shifted && killed, "null argument");
+  NOT_CAPTURED(ph->ctx);
   ScopedDevice sdv(ph->ctx);
   DevScalars h;
   int rc = ph_scalars(ph, &h, false);
@@ -800,6 +806,7 @@ int afqmc_ph_get_qr_stats(afqmc_ph ph, uint64_t* shifted, uint64_t* killed) {
 
 int afqmc_ph_set_uniforms(afqmc_ph ph, const double* u, int64_t n) {
   REQUIRE(ph && n >= 0, "invalid argument");
+  NOT_CAPTURED(ph->ctx);
   ScopedDevice sdv(ph->ctx);
   HIP_TRY(hipStreamSynchronize(ph->ctx->stream));
   ph->ubuf.release();
@@ -820,6 +827,7 @@ int afqmc_ph_set_uniforms(afqmc_ph ph, const double* u, int64_t n) {
 
 int afqmc_ph_skip_uniforms(afqmc_ph ph, uint64_t n) {
   REQUIRE(ph, "null argument");
+  NOT_CAPTURED(ph->ctx);
   ScopedDevice sdv(ph->ctx);
   DevScalars h;
   int rc = ph_scalars(ph, &h, false);
@@ -830,6 +838,7 @@ int afqmc_ph_skip_uniforms(afqmc_ph ph, uint64_t n) {
 
 int afqmc_ph_set_ET(afqmc_ph ph, double ET) {
   REQUIRE(ph, "null argument");
+  NOT_CAPTURED(ph->ctx);
   ScopedDevice sdv(ph->ctx);
   DevScalars h;
   int rc = ph_scalars(ph, &h, false);
@@ -840,6 +849,7 @@ int afqmc_ph_set_ET(afqmc_ph ph, double ET) {
 
 int afqmc_ph_get_ET(afqmc_ph ph, double* ET) {
   REQUIRE(ph && ET, "null argument");
+  NOT_CAPTURED(ph->ctx);
   ScopedDevice sdv(ph->ctx);
   DevScalars h;
   int rc = ph_scalars(ph, &h, false);
@@ -850,6 +860,7 @@ int afqmc_ph_get_ET(afqmc_ph ph, double* ET) {
 
 int afqmc_ph_log_overlap(afqmc_ph ph, afqmc_ph_walkers w, double* logO) {
   REQUIRE(ph && w && logO && w->ph == ph, "invalid argument");
+  NOT_CAPTURED(ph->ctx);
   ScopedDevice sdv(ph->ctx);
   int rc = ph->fp32 ? ph_overlap<float>(ph, w, w->wf, false, w->alive.p) : ph_overlap<double>(ph, w, w->wf, false, w->alive.p);
   if (rc) return rc;
@@ -862,6 +873,7 @@ int afqmc_ph_log_overlap(afqmc_ph ph, afqmc_ph_walkers w, double* logO) {
 
 int afqmc_ph_background(afqmc_ph ph, afqmc_ph_walkers w, double* bg) {
   REQUIRE(ph && w && bg && w->ph == ph, "invalid argument");
+  NOT_CAPTURED(ph->ctx);
   ScopedDevice sdv(ph->ctx);
   int rc = ph->fp32 ? ph_overlap<float>(ph, w, w->wf, true, w->alive.p) : ph_overlap<double>(ph, w, w->wf, true, w->alive.p);
   if (!rc) rc = ph->fp32 ? ph_theta<float>(ph, w, w->wf, w->alive.p) : ph_theta<double>(ph, w, w->wf, w->alive.p);
@@ -882,6 +894,7 @@ int afqmc_ph_background(afqmc_ph ph, afqmc_ph_walkers w, double* bg) {
 int afqmc_ph_sample_apply(afqmc_ph ph, afqmc_ph_walkers w, const double* aux, const double* force, double* sample_logw,
                           int* max_order) {
   REQUIRE(ph && w && aux && force && w->ph == ph, "invalid argument");
+  NOT_CAPTURED(ph->ctx);
   ScopedDevice sdv(ph->ctx);
   hipStream_t s = ph->ctx->stream;
   const int G = ph->G;
@@ -924,6 +937,7 @@ int afqmc_ph_sample_apply(afqmc_ph ph, afqmc_ph_walkers w, const double* aux, co
 
 int afqmc_ph_sample_matrix(afqmc_ph ph, afqmc_ph_walkers w, double* M) {
   REQUIRE(ph && w && M && w->ph == ph, "invalid argument");
+  NOT_CAPTURED(ph->ctx);
   ScopedDevice sdv(ph->ctx);
   HIP_TRY(hipStreamSynchronize(ph->ctx->stream));
   const size_t n = (size_t)ph->L * ph->L * w->nw;
@@ -939,6 +953,7 @@ int afqmc_ph_sample_matrix(afqmc_ph ph, afqmc_ph_walkers w, double* M) {
 
 int afqmc_ph_taylor_orders(afqmc_ph ph, afqmc_ph_walkers w, int* orders) {
   REQUIRE(ph && w && orders, "null argument");
+  NOT_CAPTURED(ph->ctx);
   ScopedDevice sdv(ph->ctx);
   HIP_TRY(hipStreamSynchronize(ph->ctx->stream));
   HIP_TRY(hipMemcpy(orders, ph->orders.p, sizeof(int) * w->nw, hipMemcpyDeviceToHost));
@@ -947,6 +962,7 @@ int afqmc_ph_taylor_orders(afqmc_ph ph, afqmc_ph_walkers w, int* orders) {
 
 int afqmc_ph_onebody(afqmc_ph ph, afqmc_ph_walkers w, int which) {
   REQUIRE(ph && w && w->ph == ph, "invalid argument");
+  NOT_CAPTURED(ph->ctx);
   REQUIRE(which >= 0 && which <= 2, "which must be 0, 1 or 2");
   ScopedDevice sdv(ph->ctx);
   int rc = ph->fp32 ? ph_onebody<float>(ph, w, which, w->wf, w->alive.p) : ph_onebody<double>(ph, w, which, w->wf, w->alive.p);
@@ -958,6 +974,7 @@ int afqmc_ph_onebody(afqmc_ph ph, afqmc_ph_walkers w, int which) {
 
 int afqmc_ph_stabilize(afqmc_ph ph, afqmc_ph_walkers w) {
   REQUIRE(ph && w && w->ph == ph, "invalid argument");
+  NOT_CAPTURED(ph->ctx);
   ScopedDevice sdv(ph->ctx);
   int rc = ph_stabilize_impl(ph, w);
   if (rc) return rc;
@@ -967,13 +984,14 @@ int afqmc_ph_stabilize(afqmc_ph ph, afqmc_ph_walkers w) {
 
 int afqmc_ph_step(afqmc_ph ph, afqmc_ph_walkers w, double* force_out, double* aux_out) {
   REQUIRE(ph && w && w->ph == ph, "invalid argument");
+  NOT_CAPTURED(ph->ctx);
   ScopedDevice sdv(ph->ctx);
   return PH_DISPATCH(ph, ph_step_impl, ph, w, force_out, aux_out);
 }
 
 int afqmc_ph_pop_control(afqmc_ph ph, afqmc_ph_walkers w, double* weights_out, int* table_out, double* stats) {
   REQUIRE(ph && w && w->ph == ph, "invalid argument");
-  REQUIRE(!capturing() || (!weights_out && !table_out && !stats), "a captured comb cannot return outputs");
+  REQUIRE(!captured_on(ph->ctx) || (!weights_out && !table_out && !stats), "a captured comb cannot return outputs");
   ScopedDevice sdv(ph->ctx);
   int rc = PH_DISPATCH(ph, ph_pop_control_impl, ph, w, weights_out, table_out, stats);
   if (rc) return rc;
@@ -983,6 +1001,8 @@ int afqmc_ph_pop_control(afqmc_ph ph, afqmc_ph_walkers w, double* weights_out, i
 
 int afqmc_ph_measure(afqmc_ph ph, afqmc_ph_walkers w) {
   REQUIRE(ph && w && w->ph == ph, "invalid argument");
+  REQUIRE(!captured_on(ph->ctx) || !ph->onebody_log[2],
+          "the Taylor series of exp(A) W cannot be captured (its length depends on the walkers)");
   ScopedDevice sdv(ph->ctx);
   int rc = PH_DISPATCH(ph, ph_measure_impl, ph, w);
   if (rc) return rc;
@@ -992,6 +1012,7 @@ int afqmc_ph_measure(afqmc_ph ph, afqmc_ph_walkers w) {
 
 int afqmc_ph_energy(afqmc_ph ph, double* out, double* bg_num, double* ex_num) {
   REQUIRE(ph && out, "null argument");
+  NOT_CAPTURED(ph->ctx);
   ScopedDevice sdv(ph->ctx);
   DevScalars h;
   int rc = ph_scalars(ph, &h, false);

@@ -67,6 +67,8 @@ inline void capture_note_real(const int* real) {
 inline void capture_note_call(afqmc_ctx c, std::function<int()> call) {
   if (captured_on(c)) g_capture->calls.push_back(std::move(call));
 }
+// the same for work on context c only; other contexts run as ever
+#define NOT_CAPTURED(c) REQUIRE(!captured_on(c), "%s cannot be recorded into a graph (it synchronises)", __func__)
 #define NOT_CAPTURING() REQUIRE(!capturing(), "%s cannot be recorded into a graph (it synchronises)", __func__)
 
 struct GraphPair {

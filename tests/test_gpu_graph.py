@@ -343,3 +343,35 @@ def test_graph_launch_returns_before_the_work_is_done():
         t2 = time.perf_counter()
         assert t1 - t0 < 0.5 * (t2 - t0), (theta, t1 - t0, t2 - t0)
     g.close()
+
+
+def test_phaseless_calls_that_synchronise_leave_a_capture_whole():
+    """Phaseless calls that synchronise are refused before they record anything: the capture goes on, the
+    walkers stay as they were, and contexts outside the capture run as ever."""
+    from tests.test_gpu_ph import make_case
+    c = Context(0)
+    cp, cw = make(c, 4, 4, 5, 4.0)
+    _, dm, _, prop, ws, *_ = make_case(seed=4)  # on the shared context
+    for which, alpha in ((0, 0.05), (2, -0.025)):
+        prop.set_onebody(which, *dm.log_exp_minus_alpha_k(alpha), True)
+    before, counter = ws.download(), prop.counter()
+    c.capture_begin(members=[ctx()])
+    for call in (lambda: prop.step(ws), lambda: prop.stabilize(ws), lambda: prop.onebody(ws, 0), lambda: prop.measure(ws),
+                 lambda: prop.log_overlap(ws), lambda: prop.energy(), lambda: prop.pop_control(ws, record=True),
+                 lambda: prop.set_seed(3), lambda: ws.download()):
+        with pytest.raises(Exception, match="captured|recorded into a graph"):
+            call()
+    cp.step(cw)
+    g = c.capture_end()
+    n = g.nodes()
+    g.launch()
+    c.synchronize()
+    same(before, ws.download())
+    assert prop.counter() == counter
+    g.close()
+    c.capture_begin()  # without the shared context
+    cp.step(cw)
+    prop.step(ws)
+    g = c.capture_end()
+    assert prop.counter() > counter and g.nodes() in (n - 1, n, n + 1)
+    g.close()
