@@ -145,6 +145,7 @@ SIGNATURES = {
                                    _dp, _dp, C.c_int, C.c_int, C.c_int, _dp]),
     "afqmc_test_real_gemm": (C.c_int, [_vp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _dp, _dp, _dp, C.c_int,
                                        C.c_int, _dp]),
+    "afqmc_test_ph_real_products": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int]),
     "afqmc_test_walker_panel": (C.c_int, [_vp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _dp, _dp, C.c_int, _ip,
                                           _dp]),
     "afqmc_test_gj_inverse": (C.c_int, [_vp, C.c_int, C.c_int, C.c_int, _dp, _dp, _dp, _ip]),

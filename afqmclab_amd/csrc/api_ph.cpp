@@ -106,6 +106,23 @@ bool ph_traces(afqmc_ph ph) {
   return ph->real_half != 0;
 }
 
+// bg[g][w] (+)= sum_ij A_g(i, j) X_w(i, j): one product over K = L Ns
+RealGemmArgs background_args(int G, int nw, long long K) {
+  RealGemmArgs r;
+  memset(&r, 0, sizeof(r));
+  r.M = G; r.N = nw; r.K = (int)K; r.op_t = 1;
+  r.lda = K; r.ldb = K; r.ldc = G;
+  r.alpha = 1.0;
+  return r;
+}
+
+// whether the real products take vectors of these sizes (their offsets are 32-bit); beyond, real vectors
+// stay complex numbers and take the complex products
+bool real_products_ok(bool fp32, int L, int Ns, int G) {
+  const RealGemmArgs r = background_args(G, 1, (long long)L * Ns);
+  return fp32 ? real_gemm_ok<float>(r) : real_gemm_ok<double>(r);
+}
+
 GemmArgs gbase() {
   GemmArgs a;
   memset(&a, 0, sizeof(a));
@@ -163,13 +180,11 @@ int ph_background(afqmc_ph ph, afqmc_ph_walkers w) {
   for (int sp = 0; sp < 2; ++sp) {
     const long long K = (long long)ph->L * ph->Ns[sp];
     if (ph->real_half) {  // 0.73 ms a spin at G = 1600, 1024 walkers and K = 8000, 1.00 as complex products
-      RealGemmArgs r;
-      memset(&r, 0, sizeof(r));
-      r.M = ph->G; r.N = w->nw; r.K = (int)K; r.op_t = 1;
-      r.A = ph->Ahalf[sp].p; r.lda = K;
-      r.B = ph->X[sp].p; r.ldb = K;
-      r.C = ph->bgbuf.p; r.ldc = ph->G;
-      r.alpha = 1.0; r.beta_one = sp;
+      RealGemmArgs r = background_args(ph->G, w->nw, K);
+      r.A = ph->Ahalf[sp].p;
+      r.B = ph->X[sp].p;
+      r.C = ph->bgbuf.p;
+      r.beta_one = sp;
       int rc = launch_real_gemm<T>(r, ph->ctx->stream);
       if (rc) return rc;
       continue;
@@ -556,7 +571,7 @@ int afqmc_ph_create(afqmc_ctx ctx, const afqmc_ph_desc* d, afqmc_ph* out) {
     }
   }
   const double* hr[2] = {d->half_rot_up, d->half_rot_dn};
-  ph->real_half = 1;
+  ph->real_half = real_products_ok(ph->fp32, L, ph->Ns[0], G) && real_products_ok(ph->fp32, L, ph->Ns[1], G);
   for (int sp = 0; sp < 2 && ph->real_half; ++sp)
     for (long long e = 0, n = (long long)L * ph->Ns[sp] * G; e < n && ph->real_half; ++e)
       if (hr[sp][2 * e + 1] != 0.0) ph->real_half = 0;
@@ -1050,6 +1065,10 @@ int afqmc_ph_adjust_ET(afqmc_ph ph) {
   if (rc) return rc;
   capture_note_call(ph->ctx, [=] { return afqmc_ph_adjust_ET(ph); });
   return 0;
+}
+
+int afqmc_test_ph_real_products(int precision, int L, int Ns, int G) {
+  return real_products_ok(precision != 0, L, Ns, G) ? 1 : 0;
 }
 
 }  // extern "C"

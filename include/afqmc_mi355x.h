@@ -391,6 +391,9 @@ int afqmc_test_zgemm(afqmc_ctx ctx, int precision, int opa, int M, int N, int K,
  * of B and scale are taken as zero */
 int afqmc_test_real_gemm(afqmc_ctx ctx, int precision, int op_t, int M, int N, int K, const double* A, const double* B,
                          const double* scale, int scale_group, int b_real, double* C);
+/* 1 where a phaseless propagator of these sizes (Ns: electrons of one spin) keeps real half-rotated vectors as
+ * real numbers, 0 where they are beyond the real products' 32-bit offsets and stay complex */
+int afqmc_test_ph_real_products(int precision, int L, int Ns, int G);
 /* per-walker products of real walkers (imaginary parts taken as zero, N <= 128): what = 1: out = W B (in place
  * on the device, B upper triangular with b_upper; dead walkers keep W), 2: out = W^T W (zero for dead walkers);
  * precision 1: FP32 walkers, FP64 products */

@@ -53,6 +53,20 @@ def test_errors_are_reported_not_fatal():
     assert b"null" in lib.afqmc_last_error()
 
 
+@pytest.mark.skipif(not os.path.exists(LIB), reason="library not built (run __graft_entry__.build())")
+def test_molecules_beyond_the_real_products_stay_complex():
+    """The real products address a tile of 128 columns of L Ns complex numbers by 32-bit byte offsets;
+    larger molecules keep complex half-rotated vectors, whose products have no such bound."""
+    from afqmclab_amd import _lib
+    ok = _lib.lib().afqmc_test_ph_real_products
+    for precision, size in ((0, 16), (1, 8)):
+        most = (2 ** 32 - 2) // size // 128  # 128 K + 16 elements of `size` bytes below 2^32 - 1
+        assert ok(precision, 200, 40, 1600) == 1 and ok(precision, 1, 1, 1) == 1
+        for L, Ns in ((most // 160, 160), (most // 97, 97)):
+            assert ok(precision, L - 1, Ns, 8) == 1
+            assert ok(precision, L + 1, Ns, 8) == 0
+
+
 EXE = os.path.join(ROOT, "afqmclab_amd", "afqmc_cp_run")
 
 
