@@ -315,7 +315,8 @@ class CPPropagator:
 
     def autotune(self, w, reps=5):
         """Time every tile shape on this walker set's propagate / overlap / Green GEMMs, keep the
-        fastest; returns (tiles, ms[3][n_tiles])."""
+        fastest; returns (tiles, ms[3][n_tiles]).  A GEMM whose kernel takes no tile shape (real
+        operators, real walkers) keeps the shape that is set; its row has one time and -1."""
         n = len(self.TILES)
         t = np.zeros(3, dtype=np.int32)
         ms = np.zeros(3 * n)

@@ -335,6 +335,19 @@ int cpi::stabilize(afqmc_cp cp, afqmc_walkers w) { return stabilize_impl(cp, w);
 
 // ------------------------------------------------------------------ C entry points
 namespace {
+// whether a block's call of this role takes a tile shape
+template <typename T>
+bool takes_tile(afqmc_cp cp, afqmc_walkers w, int role) {
+  RealGemmArgs r;
+  for (int b = 0; b < cp->nblk; ++b) {
+    const bool real = role == 0   ? real_propagate<T>(cp, w, 0, w->wf, w->tmp, cp->diag_only != 0, b, w->real, &r)
+                      : role == 1 ? real_overlap<T>(cp, w, w->wf, b, w->real, &r)
+                                  : real_green(cp, b, w->real);
+    if (!real) return true;
+  }
+  return false;
+}
+
 template <typename T>
 int tune_role(afqmc_cp cp, afqmc_walkers w, int role, int reps, double* ms_row) {
   hipStream_t s = cp->ctx->stream;
@@ -344,10 +357,12 @@ int tune_role(afqmc_cp cp, afqmc_walkers w, int role, int reps, double* ms_row) 
   double best = 1e300;
   int best_tile = cp->tile[role];
   int rc = 0;
+  const bool tiled = takes_tile<T>(cp, w, role);
   for (int t = 0; t < GEMM_TILE_COUNT && !rc; ++t) {
     ms_row[t] = -1.0;
     if (role == 2 && !gemm_tile_green(t)) continue;
-    cp->tile[role] = t;
+    if (!tiled && t > 0) continue;  // one kernel: timed once, and the shape set for complex walkers stays
+    if (tiled) cp->tile[role] = t;
     auto run = [&]() {
       // each role reads the walkers and writes only workspace (tmp, overlaps, Green partials)
       if (role == 0) return propagate_gemm<T>(cp, w, 0, w->wf, w->tmp, cp->diag_only != 0, w->real);
@@ -362,7 +377,7 @@ int tune_role(afqmc_cp cp, afqmc_walkers w, int role, int reps, double* ms_row) 
     float ms = 0.f;
     hipEventElapsedTime(&ms, e0, e1);
     ms_row[t] = ms / reps;
-    if (ms_row[t] < best) { best = ms_row[t]; best_tile = t; }
+    if (tiled && ms_row[t] < best) { best = ms_row[t]; best_tile = t; }
   }
   cp->tile[role] = best_tile;
   hipEventDestroy(e0);

@@ -162,6 +162,30 @@ int upload_real_operators(afqmc_cp cp, const double* phiT, const double* const* 
   return 0;
 }
 
+// Which of block b's products take a real kernel.  real: the imaginary parts of wf are zero.  The
+// kernels of the others take the tile shapes afqmc_cp_s::tile.
+template <typename T>
+bool real_overlap(afqmc_cp cp, afqmc_walkers w, DevBuf<char>* wf, int b, int real, RealGemmArgs* r) {
+  memset(r, 0, sizeof(*r));
+  r->M = cp->Nb[b]; r->N = cp->Nb[b] * w->nw; r->K = cp->Mb[b]; r->op_t = 1; r->alpha = 1.0; r->b_real = real;
+  r->A = cp->phiTr[b]; r->lda = cp->Mb[b];
+  r->B = wf[b].p; r->ldb = cp->Mb[b];
+  r->C = cp->ovl[b].p; r->ldc = cp->Nb[b];
+  return cp->real_phi && real_gemm_ok<T>(*r);
+}
+template <typename T>
+bool real_propagate(afqmc_cp cp, afqmc_walkers w, int which, DevBuf<char>* in, DevBuf<char>* out, bool scaled, int b,
+                    int real, RealGemmArgs* r) {
+  memset(r, 0, sizeof(*r));
+  r->M = cp->Mb[b]; r->N = cp->Nb[b] * w->nw; r->K = cp->Mb[b]; r->alpha = 1.0; r->b_real = real;
+  r->A = cp->expKr[which][b]; r->lda = cp->Mb[b];
+  r->B = in[b].p; r->ldb = cp->Mb[b];
+  r->C = out[b].p; r->ldc = cp->Mb[b];
+  if (scaled) { r->scale = cp->scale[b].p; r->scale_group = cp->Nb[b]; r->scale_strideG = cp->Mb[b]; }
+  return cp->real_expk[which] && !(std::is_same<T, float>::value && cp->split_bf16) && real_gemm_ok<T>(*r);
+}
+inline bool real_green(afqmc_cp cp, int b, int real) { return real && cp->Nb[b] <= WALKER_PANEL_NMAX; }
+
 // overlap O_b = phiT_b^H W_b for all walkers ("giant" GEMM with shared A).  real: the imaginary
 // parts of wf are zero.  A real trial takes real products (two per complex B element, one per
 // real one, against three in FP32 and four in FP64).
@@ -170,18 +194,11 @@ int overlap_gemm(afqmc_cp cp, afqmc_walkers w, DevBuf<char>* wf, int real = 0) {
   GroupFork fork;  // the blocks are independent: a grouped call launches them together
   for (int b = 0; b < cp->nblk; ++b) {
     fork.branch();
-    if (cp->real_phi) {
-      RealGemmArgs r;
-      memset(&r, 0, sizeof(r));
-      r.M = cp->Nb[b]; r.N = cp->Nb[b] * w->nw; r.K = cp->Mb[b]; r.op_t = 1; r.alpha = 1.0; r.b_real = real;
-      r.A = cp->phiTr[b]; r.lda = cp->Mb[b];
-      r.B = wf[b].p; r.ldb = cp->Mb[b];
-      r.C = cp->ovl[b].p; r.ldc = cp->Nb[b];
-      if (real_gemm_ok<T>(r)) {
-        int rc = launch_real_gemm<T>(r, cp->ctx->stream);
-        if (rc) return rc;
-        continue;
-      }
+    RealGemmArgs r;
+    if (real_overlap<T>(cp, w, wf, b, real, &r)) {
+      int rc = launch_real_gemm<T>(r, cp->ctx->stream);
+      if (rc) return rc;
+      continue;
     }
     GemmArgs a = gemm_base<T>();
     a.M = cp->Nb[b]; a.N = cp->Nb[b] * w->nw; a.K = cp->Mb[b]; a.batch = 1;
@@ -223,7 +240,7 @@ int green_gemm(afqmc_cp cp, afqmc_walkers w, DevBuf<char>* wf, const int* alive,
   GroupFork fork;  // the blocks are independent: a grouped call launches them together
   for (int b = 0; b < cp->nblk; ++b) {
     fork.branch();
-    if (real && cp->Nb[b] <= WALKER_PANEL_NMAX) {
+    if (real_green(cp, b, real)) {
       WalkerPanelArgs g;
       memset(&g, 0, sizeof(g));
       g.M = cp->Mb[b]; g.N = cp->Nb[b]; g.nw = w->nw;
@@ -262,19 +279,11 @@ int propagate_gemm(afqmc_cp cp, afqmc_walkers w, int which, DevBuf<char>* in, De
   GroupFork fork;  // the blocks are independent: a grouped call launches them together
   for (int b = 0; b < cp->nblk; ++b) {
     fork.branch();
-    if (cp->real_expk[which] && !(std::is_same<T, float>::value && cp->split_bf16)) {
-      RealGemmArgs r;
-      memset(&r, 0, sizeof(r));
-      r.M = cp->Mb[b]; r.N = cp->Nb[b] * w->nw; r.K = cp->Mb[b]; r.alpha = 1.0; r.b_real = real;
-      r.A = cp->expKr[which][b]; r.lda = cp->Mb[b];
-      r.B = in[b].p; r.ldb = cp->Mb[b];
-      r.C = out[b].p; r.ldc = cp->Mb[b];
-      if (scaled) { r.scale = cp->scale[b].p; r.scale_group = cp->Nb[b]; r.scale_strideG = cp->Mb[b]; }
-      if (real_gemm_ok<T>(r)) {
-        int rc = launch_real_gemm<T>(r, cp->ctx->stream);
-        if (rc) return rc;
-        continue;
-      }
+    RealGemmArgs r;
+    if (real_propagate<T>(cp, w, which, in, out, scaled, b, real, &r)) {
+      int rc = launch_real_gemm<T>(r, cp->ctx->stream);
+      if (rc) return rc;
+      continue;
     }
     GemmArgs a = gemm_base<T>();
     a.M = cp->Mb[b]; a.N = cp->Nb[b] * w->nw; a.K = cp->Mb[b]; a.batch = 1;

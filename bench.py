@@ -62,6 +62,17 @@ def flops_per_walker_step(Ls, nup, ndn, mgs, pop, meas):
     return 2.0 * (step + qr + comb + measure), 2.0 * sum(Ls * Ls * n for n in (nup, ndn))
 
 
+def tile_names(tiles, ms):
+    """The autotuned shapes by name, None for a GEMM whose kernel takes none (real operators or walkers)."""
+    from afqmclab_amd.cp import CPPropagator
+    return [CPPropagator.TILES[t] if np.any(row[1:] >= 0) else None for t, row in zip(tiles, ms)]
+
+
+def tile_numbers(names):
+    from afqmclab_amd.cp import CPPropagator
+    return [0 if t is None else CPPropagator.TILES.index(t) for t in names]
+
+
 def timed_window(thermal, warmup, steps, pop):
     """First step of the timed window: after the thermal (ET-adjust) phase and `warmup` more steps,
     moved on (never back) so that the window holds a comb when it is shorter than the comb period
@@ -93,8 +104,7 @@ def run_path(ctx, model, phi, nup, precision, nw, steps, warmup, seed, sched, ke
     prop.skip_uniforms(model.L)
     prop.onebody(ws, 1)
     # GEMM tile shapes picked by the autotuner on these walkers' own shapes (state unchanged)
-    tiles, _ = prop.autotune(ws, reps=5)
-    tiles = [CPPropagator.TILES[t] for t in tiles]
+    tiles = tile_names(*prop.autotune(ws, reps=5))
     ctx.synchronize()
     idx = [0, 0]
     counts = {"measure": 0, "qr": 0, "comb": 0}
@@ -176,7 +186,7 @@ def precision_replay(ctx, model, phi, nup, nw, sched, seed, thermal, nsteps, til
                      forceCap=1.5, mgsStep=sched["mgs"], popControlStep=sched["pop"], ET=-10.0)
         prop = CPPropagator(ctx, model, m, phi, nup=nup, spin_blocks=True, precision=precision, max_walkers=nw)
         if tiles and precision == 1:
-            prop.set_tiles(*[CPPropagator.TILES.index(t) for t in tiles])
+            prop.set_tiles(*tile_numbers(tiles))
         prop.set_ET(m.ET)
         ws = prop.walkers(nw)
         ws.set_from_trial()
@@ -326,8 +336,7 @@ def run_hetero(instances, nw, steps, seed, mode, group_tiles=(0, 0, 0)):
         sets.append((prop, ws))
     if mode == "graph" or (mode == "grouped" and min(group_tiles) < 0):
         for prop, ws in sets:
-            t, _ = prop.autotune(ws, reps=3)
-            tiles.append([CPPropagator.TILES[k] for k in t])
+            tiles.append(tile_names(*prop.autotune(ws, reps=3)))
     grp = CPGroup(sets, tiles=group_tiles) if mode == "grouped" else None
     if grp is not None and min(group_tiles) >= 0:
         tiles = [CPPropagator.TILES[k] for k in group_tiles]
@@ -422,14 +431,14 @@ def run_bp_leg(ctx, model, phi, nup, nw, nbp, skip, nmeas, seed, tiles=None):
     nbp recorded steps, nmeas measurements every skip steps.  Each measurement is timed between
     stream synchronisations; the estimates are the back-propagated energy and double occupancy.
     `tiles` (propagate, overlap, Green tile names) are the main path's tuned GEMM tiles."""
-    from afqmclab_amd.cp import AfqmcConstraintPathBP, BPMethod, CPPropagator
+    from afqmclab_amd.cp import AfqmcConstraintPathBP, BPMethod
     Ls = model.L
     m = BPMethod(dt=0.005, thermalSize=40, writeNumber=1, measureNumberPerWrite=nmeas, measureSkipStep=skip,
                  walkerSizePerThread=nw, decompType="densitySpin", mgsStep=10, popControlStep=40, ETAdjustStep=10,
                  ETAdjustMaxSize=40, backPropagationStep=nbp, seed=seed)
     drv = AfqmcConstraintPathBP(ctx, model, m, phi, nup=nup, spin_blocks=True, precision=1)
     if tiles:
-        drv.prop.set_tiles(*[CPPropagator.TILES.index(t) for t in tiles])
+        drv.prop.set_tiles(*tile_numbers(tiles))
     times = []
     measure = drv.bp.measure
 
@@ -721,9 +730,12 @@ def main():
         grouped = run_hetero(inst, 256, args.hetero_steps, args.seed, "grouped", tuple(args.hetero_tiles))
         log(f"[bench]   grouped launches, one graph per 10-step block: {grouped['walker_steps_per_s']:.0f} "
             f"walker-steps/s, {grouped['graph_nodes']} graph nodes per block")
-        tuned = run_hetero(inst, 256, args.hetero_steps, args.seed, "grouped", (-1, -1, -1))
-        log(f"[bench]   grouped launches with each instance's autotuned tiles: {tuned['walker_steps_per_s']:.0f} "
-            f"walker-steps/s, {tuned['graph_nodes']} graph nodes per block")
+        # each instance's own tile shapes in the group, where any of its GEMMs takes one
+        tiled = any(t for names in graph["tiles"] for t in names)
+        tuned = run_hetero(inst, 256, args.hetero_steps, args.seed, "grouped", (-1, -1, -1)) if tiled else grouped
+        if tiled:
+            log(f"[bench]   grouped launches with each instance's autotuned tiles: {tuned['walker_steps_per_s']:.0f} "
+                f"walker-steps/s, {tuned['graph_nodes']} graph nodes per block")
         same = all(np.allclose(a, b, rtol=1e-12, atol=0) for a, b in zip(eager["logo"], graph["logo"]))
         same_grouped = all(np.array_equal(a, b) for a, b in zip(eager["logo"], grouped["logo"]))
         same_tuned = all(np.array_equal(a, b) for a, b in zip(eager["logo"], tuned["logo"]))
@@ -736,11 +748,13 @@ def main():
             "steps": args.hetero_steps,
             "per_instance_launches": {"walker_steps_per_s": eager["walker_steps_per_s"], "seconds": eager["elapsed"]},
             "graph_autotuned": {"walker_steps_per_s": graph["walker_steps_per_s"], "seconds": graph["elapsed"],
-                                "graph_nodes_per_block": graph["graph_nodes"], "tiles": graph["tiles"]},
+                                "graph_nodes_per_block": graph["graph_nodes"], "tiles": graph["tiles"] if tiled else None},
             "grouped_graph": {"walker_steps_per_s": grouped["walker_steps_per_s"], "seconds": grouped["elapsed"],
-                              "graph_nodes_per_block": grouped["graph_nodes"], "tiles": grouped["tiles"]},
+                              "graph_nodes_per_block": grouped["graph_nodes"],
+                              "tiles": grouped["tiles"] if tiled else None},
             "grouped_graph_other_tiles": {"walker_steps_per_s": tuned["walker_steps_per_s"],
-                                          "graph_nodes_per_block": tuned["graph_nodes"], "tiles": tuned["tiles"]},
+                                          "graph_nodes_per_block": tuned["graph_nodes"],
+                                          "tiles": tuned["tiles"]} if tiled else None,
             "speedup_graph": graph["walker_steps_per_s"] / eager["walker_steps_per_s"],
             "speedup_grouped": grouped["walker_steps_per_s"] / eager["walker_steps_per_s"],
             # algorithmic flops of all instances per step (spin-block form, QR every 10, comb every

@@ -140,7 +140,11 @@ int afqmc_cp_get_ET(afqmc_cp cp, double* ET);
  * 32-deep K tile, 8 = 128x128 and 9 = 256x64 (8 waves), 10 = 64x128, with a 16-deep K tile (the Green
  * GEMM takes shapes 0, 1, 4, 5, 7, 8 and 9).  autotune times every shape on the walker set's
  * own buffers (reps launches each), keeps the fastest and returns the choices in tiles (3) and the
- * times in ms (3 x 11, ms per launch, -1 = not applicable).  Every shape gives bit-identical results. */
+ * times in ms (3 x 11, ms per launch, -1 = not applicable).  Every shape gives bit-identical results.
+ * The shapes are those of the general kernels: with a real exp(-dt K) or a real trial the propagation
+ * and the overlap, and for real walkers of at most 128 columns a block the Green's function, take kernels of
+ * one shape.  autotune then leaves the shape set for that GEMM alone and gives that kernel's time
+ * in ms[0], the rest of its row -1. */
 int afqmc_cp_set_tiles(afqmc_cp cp, const int* tiles);
 int afqmc_cp_autotune(afqmc_cp cp, afqmc_walkers w, int reps, int* tiles, double* ms);
 

@@ -60,11 +60,13 @@ def block_of_work(prop, ws):
     prop.measure(ws)
 
 
+@pytest.mark.parametrize("phases", [False, True])
 @pytest.mark.parametrize("precision", [0, 1])
-def test_every_tile_shape_gives_the_same_step(precision):
+def test_every_tile_shape_gives_the_same_step(precision, phases):
+    """(Complex operators take the shapes; real ones, whose kernels have one shape, ignore them.)"""
     ref = None
     for t in range(len(CPPropagator.TILES)):
-        prop, ws = make(ctx(), 4, 4, 5, 4.0, precision=precision)
+        prop, ws = make(ctx(), 4, 4, 5, 4.0, precision=precision, phases=phases)
         prop.set_tiles(propagate=t, overlap=t, green=t if t in GREEN_TILES else 0)
         for _ in range(2):
             prop.step(ws)
@@ -78,9 +80,10 @@ def test_every_tile_shape_gives_the_same_step(precision):
         prop.close()
 
 
-def test_autotune_keeps_state_and_results():
-    prop_a, ws_a = make(ctx(), 6, 6, 13, 4.0, precision=1, nw=64)
-    prop_b, ws_b = make(ctx(), 6, 6, 13, 4.0, precision=1, nw=64)
+@pytest.mark.parametrize("phases", [False, True])
+def test_autotune_keeps_state_and_results(phases):
+    prop_a, ws_a = make(ctx(), 6, 6, 13, 4.0, precision=1, nw=64, phases=phases)
+    prop_b, ws_b = make(ctx(), 6, 6, 13, 4.0, precision=1, nw=64, phases=phases)
     before = ws_a.download()
     tiles, ms = prop_a.autotune(ws_a, reps=3)
     after = ws_a.download()
@@ -90,10 +93,32 @@ def test_autotune_keeps_state_and_results():
     assert tiles.shape == (3,) and all(0 <= t < nt for t in tiles) and tiles[2] in GREEN_TILES
     assert ms.shape == (3, nt) and np.all(ms[:, 0] > 0)
     assert all(ms[2, t] == -1.0 for t in range(nt) if t not in GREEN_TILES)
+    if phases:
+        assert np.all(ms[:2] > 0) and all(ms[2, t] > 0 for t in GREEN_TILES)
+        assert all(ms[r, t] == np.min(ms[r][ms[r] > 0]) for r, t in enumerate(tiles))
     for _ in range(3):
         prop_a.step(ws_a)
         prop_b.step(ws_b)
     same(state(prop_a, ws_a), state(prop_b, ws_b))
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_autotune_leaves_the_shapes_that_no_kernel_takes(precision):
+    """Real walkers: three kernels of one shape, timed once, and the shapes set for complex walkers stay.
+    Complex walkers on real operators: the Green GEMM alone is tuned."""
+    prop, ws = make(ctx(), 6, 6, 13, 4.0, precision=precision, nw=64)
+    nt = len(CPPropagator.TILES)
+    own = (6, 3, 7)
+    prop.set_tiles(*own)
+    tiles, ms = prop.autotune(ws, reps=2)
+    assert tuple(tiles) == own
+    assert np.all(ms[:, 0] > 0) and np.all(ms[:, 1:] == -1.0)
+    wf, lw, _ = ws.download()
+    wf[:, :, 0] *= np.exp(0.6j)
+    ws.upload(wf, lw)
+    tiles, ms = prop.autotune(ws, reps=2)
+    assert tuple(tiles[:2]) == own[:2] and np.all(ms[:2, 0] > 0) and np.all(ms[:2, 1:] == -1.0)
+    assert all((ms[2, t] > 0) == (t in GREEN_TILES) for t in range(nt)) and ms[2, tiles[2]] == np.min(ms[2][ms[2] > 0])
 
 
 @pytest.mark.parametrize("blocks", [True, False])
