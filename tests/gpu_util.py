@@ -22,12 +22,17 @@ def ctx():
     return _CTX
 
 
+def site_phases(L, step=0.37):
+    """A phase for each of the 2 L rows (the same for both spins)."""
+    a = step * np.arange(L) ** 2 % (2 * np.pi)
+    return np.exp(1j * np.concatenate([a, a]))
+
+
 def gauged(model, step=0.37):
     """The model with a phase on every site: K_ij exp(i (a_i - a_j)).  Operators, trials and walkers
     become complex (so the general kernels run); densities, energies and weights stay."""
     from afqmclab_amd.model import HubbardModel
-    a = step * np.arange(model.L) ** 2 % (2 * np.pi)
-    p = np.exp(1j * np.concatenate([a, a]))
+    p = site_phases(model.L, step)
     return HubbardModel(L=model.L, N=model.N, K=np.asfortranarray(p[:, None] * model.K * p.conj()), U=model.U)
 
 

@@ -17,7 +17,10 @@ A walker's uniforms start after those of the earlier walkers that pass the overl
 replayed by the oracle from its own offset in the host-provided list.  FP64 bar: fields exact,
 forces, walkers, log-weights and energies to 1e-10 relative.  Mixed precision: 1e-4 relative,
 and a field may differ from the oracle's only where its uniform lies within 1e-5 of the
-field's probability threshold."""
+field's probability threshold.
+
+The lattices and their trials are real, and take the kernels for real walkers; with phases on the
+sites the same workloads run on complex data and the general kernels."""
 import cmath
 import math
 
@@ -35,7 +38,7 @@ from oracle.drivers import AfqmcConstraintPath as OracleCP, CPMethod as OracleMe
 from oracle.drivers import AfqmcPhaseless as OraclePh, PhaselessMethod as OraclePhMethod  # noqa: E402
 from oracle.models import HubbardSOC, RealMaterialMoleculeMeasureFixedSD2sSD2is, synthetic_molecule  # noqa: E402
 from oracle.rng import ListStream, gaussians_from_uniforms  # noqa: E402
-from tests.gpu_util import ctx  # noqa: E402
+from tests.gpu_util import ctx, gauged, site_phases  # noqa: E402
 
 _CACHE = {}
 
@@ -72,9 +75,12 @@ def c2_workload():
     return _CACHE["c2"]
 
 
+@pytest.mark.parametrize("phases", [False, True])
 @pytest.mark.parametrize("precision", [0, 1])
-def test_hubbard16x16_step_qr_measure_match_oracle(precision):
+def test_hubbard16x16_step_qr_measure_match_oracle(precision, phases):
     model, phi = c2_workload()
+    if phases:
+        model, phi = gauged(model), site_phases(model.L)[:, None] * phi
     L, nup, nw, dt, ET = model.L, 112, 2048, 0.005, -150.0
     tol = tol_of(precision)
     method = CPMethod(dt=dt, walkerSizePerThread=nw, decompType="densitySpin", forceType="dynamicForce",
@@ -255,9 +261,11 @@ def test_phaseless_l200_step_comb_measure_match_oracle(precision):
 
 
 # ------------------------------------------------------------------ 24 heterogeneous lattices x 256 walkers
-def hetero_sets(precision, nw, ctxs):
+def hetero_sets(precision, nw, ctxs, phases=False):
     out = []
     for c, (name, model, phi, nup) in zip(ctxs, heterogeneous_hubbard_instances()):
+        if phases:
+            model, phi = gauged(model), site_phases(model.L)[:, None] * phi
         m = CPMethod(dt=0.01, walkerSizePerThread=nw, decompType="densitySpin", ET=-1.0)
         prop = CPPropagator(c, model, m, phi, nup=nup, spin_blocks=True, precision=precision, max_walkers=nw)
         prop.set_ET(-1.0)
@@ -267,13 +275,14 @@ def hetero_sets(precision, nw, ctxs):
     return out
 
 
+@pytest.mark.parametrize("phases", [False, True])
 @pytest.mark.parametrize("precision", [0, 1])
-def test_heterogeneous_batch_graph_step_matches_oracle(precision):
+def test_heterogeneous_batch_graph_step_matches_oracle(precision, phases):
     nw = 256
     tol = tol_of(precision)
     origin = Context(0)
     ctxs = [Context(0) for _ in range(24)]
-    sets = hetero_sets(precision, nw, ctxs)
+    sets = hetero_sets(precision, nw, ctxs, phases)
     rng = np.random.default_rng(13)
     us = []
     for name, model, phi, prop, ws in sets:
@@ -309,15 +318,16 @@ def test_heterogeneous_batch_graph_step_matches_oracle(precision):
         prop.close()
 
 
-def test_heterogeneous_batch_graph_replays_equal_eager_calls():
+@pytest.mark.parametrize("phases", [False, True])
+def test_heterogeneous_batch_graph_replays_equal_eager_calls(phases):
     """10 steps + QR + comb of all 24 instances as one graph (one branch per lattice), replayed
     twice with eager work between the replays, against the same calls made eagerly on identical
     propagators: log-overlaps and walkers identical."""
     nw = 256
     origin = Context(0)
     ctxs = [Context(0) for _ in range(24)]
-    gsets = hetero_sets(1, nw, ctxs)
-    esets = hetero_sets(1, nw, [ctx()] * 24)
+    gsets = hetero_sets(1, nw, ctxs, phases)
+    esets = hetero_sets(1, nw, [ctx()] * 24, phases)
     for j, (a, b) in enumerate(zip(gsets, esets)):
         a[3].set_seed(100 + j, 0)
         b[3].set_seed(100 + j, 0)
@@ -348,14 +358,15 @@ def test_heterogeneous_batch_graph_replays_equal_eager_calls():
     g.close()
 
 
+@pytest.mark.parametrize("phases", [False, True])
 @pytest.mark.parametrize("precision", [0, 1])
-def test_grouped_step_matches_oracle(precision):
+def test_grouped_step_matches_oracle(precision, phases):
     """One grouped step of the 24 instances (every kernel of a phase launched once over all of
     them) against the oracle's step of one sampled walker per instance."""
     nw = 256
     tol = tol_of(precision)
     c = Context(0)
-    sets = hetero_sets(precision, nw, [c] * 24)
+    sets = hetero_sets(precision, nw, [c] * 24, phases)
     rng = np.random.default_rng(29)
     us = []
     for name, model, phi, prop, ws in sets:
@@ -386,9 +397,10 @@ def test_grouped_step_matches_oracle(precision):
         prop.close()
 
 
+@pytest.mark.parametrize("phases", [False, True])
 @pytest.mark.parametrize("own_tiles", [False, True])
 @pytest.mark.parametrize("precision", [0, 1])
-def test_grouped_graph_equals_per_instance_calls(precision, own_tiles):
+def test_grouped_graph_equals_per_instance_calls(precision, own_tiles, phases):
     """Blocks of 10 grouped steps + grouped QR (+ grouped comb every other block), captured as
     graphs and replayed with eager per-instance work between the replays, against the same
     per-instance calls made eagerly on identical propagators: log-overlaps, walkers, weights and
@@ -397,8 +409,8 @@ def test_grouped_graph_equals_per_instance_calls(precision, own_tiles):
     within 400 graph nodes (600 with four shapes per GEMM)."""
     nw = 256
     c = Context(0)
-    gsets = hetero_sets(precision, nw, [c] * 24)
-    esets = hetero_sets(precision, nw, [ctx()] * 24)
+    gsets = hetero_sets(precision, nw, [c] * 24, phases)
+    esets = hetero_sets(precision, nw, [ctx()] * 24, phases)
     green_shapes = [0, 1, 4, 5]
     for j, (a, b) in enumerate(zip(gsets, esets)):
         a[3].set_seed(300 + j, 0)
@@ -432,7 +444,7 @@ def test_grouped_graph_equals_per_instance_calls(precision, own_tiles):
         group_block(comb)
         graphs[comb] = c.capture_end()
     nodes = graphs[False].nodes()
-    print(f"[c4 grouped] precision={precision} own_tiles={own_tiles}: {nodes} graph nodes per 10-step "
+    print(f"[c4 grouped] precision={precision} own_tiles={own_tiles} phases={phases}: {nodes} graph nodes per 10-step "
           f"block, {grp.table_count()} argument tables", flush=True)
     assert nodes <= (600 if own_tiles else 400)
     for rep in range(4):

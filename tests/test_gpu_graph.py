@@ -121,11 +121,12 @@ def test_autotune_leaves_the_shapes_that_no_kernel_takes(precision):
     assert all((ms[2, t] > 0) == (t in GREEN_TILES) for t in range(nt)) and ms[2, tiles[2]] == np.min(ms[2][ms[2] > 0])
 
 
+@pytest.mark.parametrize("phases", [False, True])
 @pytest.mark.parametrize("blocks", [True, False])
-def test_graph_replays_match_eager_calls(blocks):
+def test_graph_replays_match_eager_calls(blocks, phases):
     c_graph, c_eager = Context(0), Context(0)
-    pg, wg = make(c_graph, 4, 4, 5, 4.0, blocks=blocks)
-    pe, we = make(c_eager, 4, 4, 5, 4.0, blocks=blocks)
+    pg, wg = make(c_graph, 4, 4, 5, 4.0, blocks=blocks, phases=phases)
+    pe, we = make(c_eager, 4, 4, 5, 4.0, blocks=blocks, phases=phases)
     c_graph.capture_begin()
     block_of_work(pg, wg)
     g = c_graph.capture_end()
@@ -143,13 +144,14 @@ def test_graph_replays_match_eager_calls(blocks):
     g.close()
 
 
-def test_group_graph_of_independent_lattices_matches_per_instance_calls():
+@pytest.mark.parametrize("phases", [False, True])
+def test_group_graph_of_independent_lattices_matches_per_instance_calls(phases):
     shapes = [(4, 4, 5, 4.0), (6, 6, 13, 3.0), (6, 4, 9, 6.0)]
     origin = Context(0)
     gctx = [Context(0) for _ in shapes]
     ectx = Context(0)
-    graph_sets = [make(c, *s, precision=1, seed=11 + i) for i, (c, s) in enumerate(zip(gctx, shapes))]
-    eager_sets = [make(ectx, *s, precision=1, seed=11 + i) for i, s in enumerate(shapes)]
+    graph_sets = [make(c, *s, precision=1, seed=11 + i, phases=phases) for i, (c, s) in enumerate(zip(gctx, shapes))]
+    eager_sets = [make(ectx, *s, precision=1, seed=11 + i, phases=phases) for i, s in enumerate(shapes)]
     for p, w in graph_sets:
         p.autotune(w, reps=2)
     origin.capture_begin(members=gctx)
