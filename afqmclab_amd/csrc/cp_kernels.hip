@@ -69,7 +69,9 @@ __device__ __forceinline__ void logo_walker(const LogOArgs& a, int w) {
       if (a.info[b][w]) singular = 1;
     }
   }
-  if (singular) { re = -1e300; ang = 0.0; }
+  // A determinant beyond the largest number (an overlap that overflowed) is no weight either: whether its
+  // Gauss-Jordan ends singular, infinite or NaN depends on where the infinity sits and on the kernel.
+  if (singular || !isfinite(re) || !isfinite(ang)) { re = -1e300; ang = 0.0; }
   zd lw = a.logw[w];
   zd lo = cmk<double>(a.trial_logw.re + lw.re + re, -a.trial_logw.im + lw.im + ang);
   a.logO[w] = lo;

@@ -293,3 +293,29 @@ def test_step_head_numbers_the_alive_walkers(nw):
         assert prop.counter() == 5 + int(np.sum(al != 0)) * L
         got.append(np.where(al[:, None] != 0, aux, 0))
     assert np.array_equal(got[0][:len(got[1])], got[1])
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("nup,col", [(1, 0), (5, 0), (5, 4), (20, 19)])
+def test_walkers_whose_overlap_overflows_weigh_nothing(precision, nup, col):
+    """A walker whose overlap with the trial is beyond the largest number has no usable weight: it counts as
+    one of overlap zero (log-overlap -1e300, weight 0, killed by the comb) and leaves the others alone,
+    with real walkers and with complex ones."""
+    nx = 4 if nup < 10 else 7
+    (pr, wr), (pc, wc) = pair(nx, nx, nup, nup, False, precision, nw=4)
+    big = 3e38 if precision else 1.7e308
+    model = HubbardModel.square(nx, nx, 2 * nup, 6.0)
+    phi = spin_block_trial(model, nup, nup)
+    L = model.L
+    assert np.sum(np.abs(phi[:L, col])) > 1.2 * (3.41 / 3 if precision else 1.8 / 1.7)
+    for p, w, phase in ((pr, wr, 1.0), (pc, wc, np.exp(0.6j))):
+        wf, lw, _ = w.download()
+        good = p.log_overlap(w)
+        x = big * np.sign(phi[:L, col].real)
+        wf[2, :L, col] = x * (phase if col == 0 else 1.0)
+        w.upload(wf, lw)
+        lo = p.log_overlap(w)
+        assert lo[2].real < -1e299 and np.array_equal(lo[[0, 1, 3]], good[[0, 1, 3]])
+        weight, table, _ = p.pop_control(w, record=True)
+        assert weight[2] == 0 and np.all(weight[[0, 1, 3]] > 0) and np.all(np.isfinite(weight))
+        assert 2 not in table and np.all(w.alive() != 0)
