@@ -660,7 +660,7 @@ struct GjBK {
   static constexpr int NMAX_B = 16 * NR;
   // (FP32 storage only: with FP64 storage at 65 to 80 columns, the one size that fits, 1024
   // inversions of 72 x 72 took 0.309 ms against 0.295 without staging)
-  static constexpr bool STAGE = NRF == 2 && sizeof(T) == 4 && sizeof(E) == 16 && sizeof(cplx<T>) * NMAX_B * NMAX_B <= 104 * 1024;
+  static constexpr bool STAGE = NRF == 2 && sizeof(T) == 4 && sizeof(cplx<T>) * NMAX_B * NMAX_B <= 104 * 1024;
   __device__ static void run(const BlockIdx3& bk, const SmallDenseArgs& p);
 };
 template <typename T, typename E, int NR, int NC, int WV, int NRF, int WPEV>
@@ -668,6 +668,7 @@ __device__ __forceinline__ void GjBK<T, E, NR, NC, WV, NRF, WPEV>::run(const Blo
   constexpr int NB = 4, CPW = 4 * NC;  // panel size, columns per update wave
   constexpr int COLS = CPW * WV, FROWS = 64 * NRF;
   static_assert(16 * NR <= FROWS && NR * NC >= NRF * NB, "row capacity");
+  static_assert(sizeof(E) == 16 || NRF == 1, "real matrices of more than 64 rows take GjTK");
   const int N = p.N;
   const int NP = (N + NB - 1) / NB;
   // thread, lane and the lane's row and column in the 2-D layout: set again, opaque to the compiler,
@@ -786,27 +787,14 @@ __device__ __forceinline__ void GjBK<T, E, NR, NC, WV, NRF, WPEV>::run(const Blo
       int pr, rr, pl;
       E prv[NB];
       if constexpr (sizeof(E) == 8) {
-        // real: 32-bit keys, and the pivot row by readlanes (eight per row group, the group chosen
-        // among scalars): no LDS round trip on the chain
-        unsigned key = 0u;
-#pragma unroll
-        for (int r = 0; r < NRF; ++r) {
-          const int i = lane + 64 * r;
-          const unsigned kk = (i < N && !((used >> r) & 1u)) ? pivot_key32(y[r][q], i) : 0u;
-          key = kk > key ? kk : key;
-        }
+        // real: 32-bit keys, and the pivot row by readlanes: no LDS round trip on the chain
+        const unsigned key = (lane < N && !(used & 1u)) ? pivot_key32(y[0][q], lane) : 0u;
         const int bi = 255 - (int)(wave_max_u32(key) & 0xFFu);
         pr = (bi >= 0 && bi < N) ? bi : 0;
-        rr = pr >> 6;
-        pl = pr & 63;
+        rr = 0;
+        pl = pr;
 #pragma unroll
-        for (int q2 = 0; q2 < NB; ++q2) {
-          prv[q2] = readlane_e(y[0][q2], pl);
-          if constexpr (NRF > 1) {
-            const E v = readlane_e(y[NRF - 1][q2], pl);
-            prv[q2] = rr ? v : prv[q2];
-          }
-        }
+        for (int q2 = 0; q2 < NB; ++q2) prv[q2] = readlane_e(y[0][q2], pl);
       } else {
         unsigned long long key = 0ull;
 #pragma unroll
