@@ -122,9 +122,9 @@ int cholqr_f64(const CholQrBlock& q, hipStream_t s) {
   return refine(q, q.flag, s);
 }
 
-// 1024 walkers of 256 x 112: Gram matrix 184, factorisation 313, W R^-1 340, check 194 us, the passes
-// over the masks (empty in an ordinary run) 5 us each: 1.1 ms.  With FP64 copies of all walkers
-// and complex products the same took 4.3 ms.
+// A block of 2048 walkers of 256 x 112: Gram matrix 186, factorisation 610, W R^-1 337, check 194 us, the
+// passes over the masks (empty in an ordinary run) 5 us each: 1.4 ms (1024 walkers 0.75).  With FP64
+// copies of all walkers and complex products 2048 of them took 4.2 ms.
 int cholqr_real_f32(const CholQrBlock& q, const void* w32, void* out, void* gram32, int* mask, double check_tol,
                     hipStream_t s) {
   REQUIRE(panels(q), "real FP32 CholeskyQR: real walkers of at most %d columns", WALKER_PANEL_NMAX);

@@ -11,7 +11,7 @@
 //
 // What bounds it is the pivoting wave's serial chain (search, reciprocal, three eliminations, four times
 // a panel: some 9800 cycles at 112 columns with three matrices on a compute unit, against 2350 of
-// its matrix cores); the tiles take 2 RT registers a lane and little else, so that three matrices
+// its matrix cores; which part of the chain takes them was not measured); the tiles take 2 RT registers a lane and little else, so that three matrices
 // share a compute unit at 112 columns where the vector form fitted two.
 // FP32 storage, against GjBK with real elements: 2048 inversions of 112 columns 341 us, 364; in a group
 // of 24 x 256 matrices of mixed sizes those of 65-80 columns 240, 260; 49-64: 281, 353; 33-48: 128,

@@ -9,10 +9,10 @@
 // four k) then spread over the banks.
 //
 // Measured on MI355X (kernel trace, 2048 walkers of 256 x 112 per launch): propagation with the
-// fused HS scale 0.378 ms in FP32 and 0.971 ms in FP64 for real walkers, against 0.922 and 2.227 ms
-// for the complex kernel; overlap 0.162 and 0.401 against 0.458 and 1.075 ms.  The floor of the
+// fused HS scale 0.352 ms in FP32 and 0.971 ms in FP64 for real walkers, against 0.922 and 2.227 ms
+// for the complex kernel; overlap 0.156 and 0.401 against 0.458 and 1.075 ms.  The floor of the
 // FP32 propagation is its 0.94 GB of walkers, read and written once: 0.20 ms at the 4.75 TB/s of a
-// large copy.  Multiplying the scale and masking at the load instead of at the store cost 0.28 ms
+// large copy (0.97 GB by the counters; matrix cores busy 0.54 of the time).  Multiplying the scale and masking at the load instead of at the store cost 0.28 ms
 // (every K tile then waited for its loads before its MFMAs).
 #include "real_gemm.hpp"
 
@@ -206,6 +206,16 @@ int pick_rows(const RealGemmArgs& a, hipStream_t s) {
   // The row fragments of a tile: as few padded rows as possible, then as many rows as possible (B
   // is read once per row tile), but small tiles while the launch would leave compute units idle
   // (a grouped call launches the members' tiles together).  Every choice sums in the same order.
+  // Weighing padded rows above everything is right only where a tile of several fragments pads nothing.
+  // Real walkers, us per launch with 8 / 7 / 4 / 3 / 2 / 1 fragments, the chosen one in brackets:
+  //   propagation FP32, 2048 walkers of 100 x 44: 43 / [41] / 46 / 52 / 54 / 79
+  //                     1024 of 144 x 64:         67 / 62 / 56 / [47] / 57 / 86
+  //                     2048 of 80 x 36:          32 / 30 / 33 / 27 / 29 / [38]
+  //                     1024 of 196 x 86:         125 / 114 / 128 / 133 / 153 / [244]
+  //   propagation FP64, 1024 of 196 x 86:         345 / 315 / 276 / 280 / 253 / [346]
+  //   overlap FP32,     1024 of 256 x 112:        97 / [89] / 88 / 100 / 105 / 143
+  // 5, 11 and 13 fragments (65-80, 161-176, 193-208 rows) thus take single fragments where 16 to 22 %
+  // of padding in larger tiles would be up to twice as fast.
   constexpr int opts[6] = {8, 7, 4, 3, 2, 1};
   const long long cols = (a.N + 127) / 128;
   int best = 1;

@@ -3,8 +3,9 @@
 // of the matrix in LDS so that two matrices share a CU.
 //
 // gj_inverse_logdet: Gauss-Jordan exchange sweep with partial pivoting.  The pivot of column k
-//   is the largest |re|+|im| among rows not yet used, first index on ties, as izamax in zgetrf,
-//   so the pivots equal LU's u_kk and
+//   is the largest |re|+|im| among rows not yet used, first index on ties, as izamax in zgetrf
+//   (real matrices of up to 112 columns: the largest |x| to 2^-12, see pivot_key32; a threshold choice
+//   whose determinant and inverse are LU's up to rounding), so the pivots equal LU's u_kk and
 //   logdet = sum log|u_kk| + log(prod u_kk/|u_kk| * sign(perm)) reproduces logDeterminant
 //   (tensor_2d_common_fun.cpp:75-105).  Writes O^{-1}.
 //   Column layout: wave w owns columns w + 16c, lane l rows l + 64r, so a column and its pivot

@@ -1393,13 +1393,14 @@ int dispatch_registers(int kind, const SmallDenseArgs& a, hipStream_t s) {
     // trips of every step on the chain); the panel kernel for 33 to 48 columns (40: 0.148 against
     // 0.262 ms, four matrices per CU) and 65 to 112 (112: 2.16 against 2.34 ms; 72: 0.309 against
     // 0.343; 96: 1.72 against 1.74), where its registers allow one or two matrices per CU; the 1-D
-    // layout otherwise (64: 0.29 against 0.42 for the panel kernel, which fits two matrices per CU
-    // there against the 1-D kernel's four).  While all matrices fit the device at two per CU anyway, the
-    // panel kernel's shorter chain wins at 49 to 64 columns too (FP32 storage, 61 columns: 300
-    // matrices 58 us against 95, 512: 62 against 97, 1024: 160 against 154; FP64, 56 columns, 128
-    // matrices: 45 against 55).  The choice depends on the call's own N and batch only, so that a
-    // grouped call and the members' own calls do the same arithmetic (the panel kernel's results
-    // differ from the others' in rounding).
+    // layout otherwise.  At 49 to 64 columns the panel kernel fits two matrices per CU and the 1-D
+    // kernel four: while all matrices fit the device at two per CU the panel kernel's shorter chain wins
+    // (56 columns, panel against 1-D: FP32 storage 256 matrices 45 us against 56, 512: 55 against 88,
+    // 1024: 143 against 141, 6144: 712 against 702; FP64 47 against 56, 58 against 87, 147 against 139,
+    // 726 against 691).  The choice depends on the call's own N and batch only, so that a grouped
+    // call and the members' own calls do the same arithmetic (the panel kernel's results differ from
+    // the others' in rounding): a group whose members have up to two matrices per CU takes panels for
+    // all of them together, which costs up to 8 % of this kernel at 1024 matrices and 5 % at 6144.
     // a grouped call launches the matrices of all its members together
     const bool many = a.batch > cu_count() || grouping();
     const bool panels = a.N <= 48 || (a.N > 64 && a.N <= 112) || (a.N <= 64 && a.batch <= 2 * cu_count());

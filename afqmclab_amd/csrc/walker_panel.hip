@@ -11,9 +11,9 @@
 // operands.  Only the 16 x 16 blocks on or above the diagonal are computed, dealt out to the waves
 // in turn (at 112 columns 28 of 49), and written twice.
 //
-// Measured on MI355X (kernel trace, 2048 walkers of 256 x 112): green 0.25 ms in FP32 and 0.34 ms in
-// FP64, against 0.52 and 1.07 ms for the complex kernel's Green epilogue.  32 rows per wave spilled
-// or halved the waves in flight (0.27-0.36 and 0.35-0.48 ms).
+// Measured on MI355X (kernel trace, 2048 walkers of 256 x 112): green 0.19 ms in FP32 and 0.34 ms in
+// FP64, against 0.52 and 1.07 ms for the complex kernel's Green epilogue (matrix cores busy 0.43 and 0.50 of the
+// time).  32 rows per wave spilled or halved the waves in flight (0.27-0.36 and 0.35-0.48 ms).
 #include "walker_panel.hpp"
 
 #include "group.hpp"

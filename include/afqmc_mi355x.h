@@ -154,8 +154,9 @@ int afqmc_cp_autotune(afqmc_cp cp, afqmc_walkers w, int reps, int* tiles, double
  * mixed; not the split-BF16 propagation), no two sharing a propagator.  group_step, group_stabilize
  * and group_pop_control do what afqmc_cp_step, afqmc_cp_stabilize and afqmc_cp_pop_control (without
  * outputs) do on every member, with the same results, but launch each kernel of a phase once over
- * all members (about ten launches per step instead of ten per member), which a graph captured from
- * group calls replays.  The group's tile shapes (set_tiles, as afqmc_cp_set_tiles; 64x64 by default)
+ * all members that take it (24 lattices of 6 x 6 to 12 x 12 sites: 17 launches a step for complex walkers, 37
+ * for real ones, whose kernels come in more size classes, instead of some ten a member), which a graph
+ * captured from group calls replays.  The group's tile shapes (set_tiles, as afqmc_cp_set_tiles; 64x64 by default)
  * stand in for the members' own during its calls; a shape of -1 keeps each member's own for that
  * GEMM (members with equal shapes share a launch, each other shape adds one).  Argument tables of the grouped launches are kept
  * on the device until group_destroy (table_count: how many), so graphs captured from a group's calls
