@@ -675,6 +675,14 @@ def main():
                      "algorithmic_bytes": per_launch_bytes},
         "paths": {},
     }
+    # HBM bytes per launch of that kernel on real walkers, from the committed rocprofv3 FETCH_SIZE /
+    # WRITE_SIZE passes scaled by the same counters on a plain copy (profiles/)
+    tpath = os.path.join(ROOT, "profiles", "cp_propagate_traffic.json")
+    if os.path.exists(tpath) and r["tiles"][0] is None:
+        with open(tpath) as f:
+            tr = json.load(f)
+        if tr.get("workload_walkers") == args.walkers and tr.get("path") == main_path:
+            out["roofline"]["traffic"] = tr.get("real_gemm", {}).get("hbm_bytes_per_launch")
     if copy_cal:
         out["copy_calibration"] = copy_cal
     for p, rr in results.items():
