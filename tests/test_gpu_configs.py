@@ -405,7 +405,7 @@ def test_grouped_graph_equals_per_instance_calls(precision, own_tiles, phases):
     graphs and replayed with eager per-instance work between the replays, against the same
     per-instance calls made eagerly on identical propagators: log-overlaps, walkers, weights and
     alive flags identical.  With own_tiles the members keep different GEMM tile shapes of their
-    own (group tiles -1: one grouped launch per shape in use).  The block without the comb stays
+    own (group tiles -1: one grouped launch per shape in use; real lattices' kernels take none).  The block without the comb stays
     within 400 graph nodes (600 with four shapes per GEMM)."""
     nw = 256
     c = Context(0)
