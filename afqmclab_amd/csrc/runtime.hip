@@ -477,10 +477,14 @@ int afqmc_graph_launch(afqmc_graph g) {
       for (afqmc_ctx m : g->members) HIP_TRY(hipStreamWaitEvent(m->stream, g->ev, 0));
     }
     int rc = 0;
-    g_reissuing = true;
-    for (auto& call : g->calls)
-      if (!rc) rc = call();
-    g_reissuing = false;
+    {
+      struct Reissuing {
+        Reissuing() { g_reissuing = true; }
+        ~Reissuing() { g_reissuing = false; }
+      } reissuing;
+      for (auto& call : g->calls)
+        if (!rc) rc = call();
+    }
     for (afqmc_ctx m : g->members) {
       HIP_TRY(hipEventRecord(g->ev, m->stream));
       HIP_TRY(hipStreamWaitEvent(s, g->ev, 0));

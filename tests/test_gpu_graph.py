@@ -244,7 +244,7 @@ class Comb:
             d.put(np.full_like(d.host, -7))
 
 
-@pytest.mark.parametrize("form", ["context", "members", "group"])
+@pytest.mark.parametrize("form", ["context", "members", "group", "group on a member"])
 @pytest.mark.parametrize("precision", [0, 1])
 def test_graph_of_real_walkers_makes_all_its_calls_for_complex_ones(form, precision):
     """A graph captured while its sets are real, launched after one of them became complex: every
@@ -254,10 +254,11 @@ def test_graph_of_real_walkers_makes_all_its_calls_for_complex_ones(form, precis
     change parity between the launches)."""
     shapes = [(4, 4, 5, 4.0), (6, 4, 9, 3.0)]
     origin = Context(0)
-    gctx = [Context(0) for _ in shapes] if form == "members" else [origin] * len(shapes)
+    member = Context(0)
+    gctx = {"members": [member, Context(0)], "group on a member": [member, member]}.get(form, [origin, origin])
     gsets = [make(c, *s, precision=precision, seed=21 + i) for i, (c, s) in enumerate(zip(gctx, shapes))]
     esets = [make(ctx(), *s, precision=precision, seed=21 + i) for i, s in enumerate(shapes)]
-    grp = CPGroup(gsets) if form == "group" else None
+    grp = CPGroup(gsets) if form.startswith("group") else None
     comb = Comb(gctx[1], 500, 8)
     start = [w.download()[0] for _, w in gsets]
 
@@ -273,7 +274,7 @@ def test_graph_of_real_walkers_makes_all_its_calls_for_complex_ones(form, precis
         for p, w in sets:
             p.measure(w)
 
-    origin.capture_begin(members=gctx if form == "members" else ())
+    origin.capture_begin(members=[c for c in dict.fromkeys(gctx) if c is not origin])
     block(gsets, grp)
     comb.call()
     g = origin.capture_end()
