@@ -4,9 +4,9 @@ on sampled walkers:
 * 16 x 16 Hubbard, U = 8, 112 + 112, UHF trial, 2048 spin-block walkers: one step with
   host-provided uniforms (fields, forces, walkers, log-weights), one QR and one measurement;
 * the phaseless synthetic molecule, L = 200, 40 + 40, G = 1600, 1024 walkers: one step, one
-  QR + comb over all walkers, and one measurement whose exchange GEMM runs in walker chunks
-  (the per-walker blocks of all 1024 walkers exceed the 4 GiB chunk buffer), with the measured
-  walkers placed on both sides of chunk boundaries;
+  QR + comb over all walkers, and one measurement whose exchange GEMM (real vectors in FP64,
+  complex ones) runs in walker chunks (the per-walker blocks of all 1024 walkers exceed the 4 GiB
+  chunk buffer), with the measured walkers placed on both sides of chunk boundaries;
 * 24 heterogeneous lattices (6 x 6 to 12 x 12) x 256 walkers: one graph step of all instances
   against the oracle, and graph replays of 10 steps + QR + comb against eager calls; the same with
   grouped launches (one launch per kernel and phase over all instances) against the oracle and,
@@ -166,12 +166,19 @@ def c3_workload():
     return _CACHE["c3"]
 
 
+@pytest.mark.parametrize("phases", [False, True])
 @pytest.mark.parametrize("precision", [0, 1])
-def test_phaseless_l200_step_comb_measure_match_oracle(precision):
+def test_phaseless_l200_step_comb_measure_match_oracle(precision, phases):
+    """With a phase on every column of the trial the half-rotated vectors are complex, and the measurement's
+    exchange runs in chunks of walkers in both precisions (the real ones' traces need no chunks in FP32)."""
     om, dm = c3_workload()
     L, N, G, nw, dt, ET = 200, 40, 1600, 1024, 0.005, -150.0
     tol = tol_of(precision)
     ref = OraclePh(OraclePhMethod(dt=dt, walkerSizePerThread=nw, ET=ET), om, ListStream(np.zeros(0)))
+    if phases:
+        for wf in (ref.phiT.wfUp, ref.phiT.wfDn):
+            wf *= np.exp(0.3j * np.arange(1, N + 1))
+        ref.mixedMeasure = RealMaterialMoleculeMeasureFixedSD2sSD2is(om, ref.phiT)
     method = PhaselessMethod(dt=dt, walkerSizePerThread=nw, ET=ET)
     prop = PhaselessPropagator(ctx(), dm, method, phiT=(ref.phiT.wfUp, ref.phiT.wfDn), precision=precision,
                                max_walkers=nw)
