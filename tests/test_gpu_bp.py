@@ -16,7 +16,7 @@ from oracle.blocks import SD  # noqa: E402
 from oracle.drivers import AfqmcConstraintPathBP as OracleBP, BPMethod as OracleBPMethod  # noqa: E402
 from oracle.models import HubbardSOC  # noqa: E402
 from oracle.rng import UniformStream  # noqa: E402
-from tests.gpu_util import ctx  # noqa: E402
+from tests.gpu_util import ctx, gauged  # noqa: E402
 
 KEYS = ("den", "HNum", "KNum", "VNum", "RNum", "greenMatrixNum", "densityDensityNum", "splusSminusNum",
         "sminusSplusNum", "spairSpairNum")
@@ -79,12 +79,15 @@ def test_bp_hop_decompositions_match_oracle(decomp):
     compare_writes(dev.writes, ref.writes, 1e-9)
 
 
+@pytest.mark.parametrize("phases", [False, True])
 @pytest.mark.parametrize("mode,nup,ndn", [("dense", 5, 5), ("blocks", 5, 5), ("blocks", 6, 3)])
-def test_bp_hubbard_matches_oracle(mode, nup, ndn):
+def test_bp_hubbard_matches_oracle(mode, nup, ndn, phases):
     """4x4 Hubbard, densitySpin, diagonal site matrices: dense walkers and spin blocks (also with
-    Nup != Ndn)."""
+    Nup != Ndn), real and with phases on the sites (the general kernels)."""
     nx, ny, U = 4, 4, 4.0
     model = HubbardModel.square(nx, ny, nup + ndn, U)
+    if phases:
+        model = gauged(model)
     phi = free_electron_trial(model) if mode == "dense" else spin_block_trial(model, nup, ndn)
     kw = dict(spin_blocks=False) if mode == "dense" else dict(nup=nup, spin_blocks=True)
     seed = 2024
@@ -95,12 +98,15 @@ def test_bp_hubbard_matches_oracle(mode, nup, ndn):
     compare_writes(dev.writes, ref.writes, 1e-9)
 
 
+@pytest.mark.parametrize("phases", [False, True])
 @pytest.mark.parametrize("precision", [1, 2])
-def test_bp_mixed_precision_close_to_oracle(precision):
+def test_bp_mixed_precision_close_to_oracle(precision, phases):
     """FP32 walkers and GEMMs (precision 2: the propagation GEMMs of kets and bras in split-BF16
     products): the same run to the mixed-precision bar (energies 1e-4 relative)."""
     nx, ny, nup, ndn, U = 4, 4, 5, 5, 4.0
     model = HubbardModel.square(nx, ny, nup + ndn, U)
+    if phases:
+        model = gauged(model)
     phi = spin_block_trial(model, nup, ndn)
     seed = 7
     m = dict(dt=0.05, thermalSize=10, writeNumber=1, measureNumberPerWrite=2, measureSkipStep=4,
