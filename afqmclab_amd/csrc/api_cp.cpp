@@ -1242,6 +1242,10 @@ namespace {
 template <class F>
 int run_grouped(afqmc_cp_group g, F&& per_member) {
   REQUIRE(!grouping(), "grouped calls do not nest");
+  // a group's launches fork side streams from its context's stream: not from one that a capture has itself
+  // forked from its origin (ending such a capture has crashed inside the runtime)
+  REQUIRE(!captured_on(g->ctx) || g->ctx == g_capture->origin,
+          "a group's calls are captured on the capture's origin, not on a member context");
   ScopedDevice sd(g->ctx);
   GroupCollector c;
   c.tables = &g->tables;

@@ -47,8 +47,9 @@ int afqmc_ctx_get_timing(afqmc_ctx ctx, double* total_ms, long long* count, int 
  * nothing).  Between begin and end, the calls made on this thread are recorded instead of run:
  * afqmc_cp_step (without records), afqmc_cp_stabilize, afqmc_cp_pop_control (without outputs),
  * afqmc_cp_measure, afqmc_cp_onebody, afqmc_cp_reset_measure, afqmc_cp_adjust_ET, the calls of a group
- * of runs, afqmc_comb_noalloc, and of the phaseless calls afqmc_ph_measure (with a dense one-body
- * operator), afqmc_ph_pop_control (without outputs), afqmc_ph_reset_measure and afqmc_ph_adjust_ET.
+ * of runs (with its context as the capture's origin; on a member context they are refused),
+ * afqmc_comb_noalloc, and of the phaseless calls afqmc_ph_measure (with a dense one-body operator),
+ * afqmc_ph_pop_control (without outputs), afqmc_ph_reset_measure and afqmc_ph_adjust_ET.
  * Calls that return data to the host fail while a capture is open.  begin_group also records work issued on
  * the member contexts (one stream each; e.g. independent lattices), which become parallel
  * branches of one graph.  afqmc_graph_launch enqueues the whole graph on the origin's stream

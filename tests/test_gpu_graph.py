@@ -244,7 +244,9 @@ class Comb:
             d.put(np.full_like(d.host, -7))
 
 
-@pytest.mark.parametrize("form", ["context", "members", "group", "group on a member"])
+@pytest.mark.parametrize("form", ["context", "members", "group", pytest.param("group on a member", marks=pytest.mark.skip(
+    reason="a capture whose member stream forks a group's side streams has crashed the process in capture_end; "
+           "group calls on a member context are refused"))])
 @pytest.mark.parametrize("precision", [0, 1])
 def test_graph_of_real_walkers_makes_all_its_calls_for_complex_ones(form, precision):
     """A graph captured while its sets are real, launched after one of them became complex: every
@@ -296,6 +298,31 @@ def test_graph_of_real_walkers_makes_all_its_calls_for_complex_ones(form, precis
     g.close()
     if grp:
         grp.close()
+
+
+def test_group_calls_are_captured_on_the_origin_only():
+    """A group whose context is a member of the capture: refused before anything is recorded, and the capture
+    stays whole."""
+    origin, member = Context(0), Context(0)
+    p, w = make(member, 4, 4, 5, 4.0)
+    grp = CPGroup([(p, w)])
+    before = state(p, w)
+    origin.capture_begin(members=[member])
+    for call in (grp.step, grp.stabilize, grp.pop_control):
+        with pytest.raises(Exception, match="captured on the capture's origin"):
+            call()
+    p.onebody(w, 0)
+    g = origin.capture_end()
+    same(state(p, w), before)
+    g.launch()
+    origin.synchronize()
+    member.synchronize()
+    assert not np.array_equal(w.download()[0], before[0])
+    g.close()
+    grp.step()
+    member.synchronize()
+    assert p.counter() > before[3]
+    grp.close()
 
 
 def test_graph_with_phaseless_calls_makes_them_for_complex_walkers_too():
